@@ -58,7 +58,7 @@ def listed():
          "samples": 50},
         # NUTS draws of the stochastic-volatility model continued at a given step size
         {"name": "nuts-sv", "kind": "nuts-sv", "T": 3000, "C": 128, "samples": 10,
-         "step": 0.05},
+         "step": 0.01},
     ]
 
 
@@ -103,7 +103,7 @@ def draw(rng):
                 "C": rng.randint(1, 8), "warmup": rng.randint(30, 50),
                 "samples": rng.randint(20, 50)}
     return {"kind": "nuts-sv", "T": _log(rng, 500, 3000), "C": _log(rng, 8, 128),
-            "samples": rng.randint(5, 10), "step": 0.05}
+            "samples": rng.randint(5, 10), "step": 0.01}
 
 
 # ---- inputs ---------------------------------------------------------------------
