@@ -370,6 +370,13 @@ int nax_set_graphs(nax_sampler* h, int32_t enable);
 int nax_diagnostics(const float* d_x, int32_t chains, int32_t draws, int32_t params,
                     double* d_ess, double* d_split_rhat);
 
+/* The same with a caller's workspace (256-byte aligned device memory of
+ * nax_diagnostics_workspace() bytes), for callers with their own allocator;
+ * nax_diagnostics allocates and frees one.  0 bytes: sizes it refuses. */
+int64_t nax_diagnostics_workspace(int32_t chains, int32_t draws, int32_t params);
+int nax_diagnostics_ws(const float* d_x, int32_t chains, int32_t draws, int32_t params,
+                       double* d_ess, double* d_split_rhat, void* d_ws, int64_t ws_bytes);
+
 #ifdef __cplusplus
 }
 #endif

@@ -114,6 +114,9 @@ SIGNATURES = {
     "nax_set_graphs": (C.c_int, [C.c_void_p, C.c_int32]),
     "nax_diagnostics": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_void_p,
                                   C.c_void_p]),
+    "nax_diagnostics_workspace": (C.c_int64, [C.c_int32, C.c_int32, C.c_int32]),
+    "nax_diagnostics_ws": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, C.c_void_p,
+                                     C.c_void_p, C.c_void_p, C.c_int64]),
     "nax_kernel_timing": (C.c_int, [C.c_void_p, C.c_int32, C.POINTER(C.c_double),
                                     C.POINTER(C.c_int64)]),
 }

@@ -4,7 +4,7 @@ Same formulas as ``numpyro/diagnostics.py``: ESS by autocovariance and
 Geyer's initial monotone sequence (``diagnostics.py:101-203``), split
 Gelman-Rubin (``64-80``).  Host NumPy for arrays; ``device_diagnostics``
 computes ESS and split R-hat of draws already on the GPU with the library's
-kernel (one workgroup per parameter).
+kernels (a tile of parameters per workgroup).
 """
 import numpy as np
 
@@ -137,7 +137,11 @@ def device_diagnostics(x):
     xf = x.to(device="cuda", dtype=torch.float32).reshape(C, S, P).contiguous()
     ess = torch.empty(P, dtype=torch.float64, device="cuda")
     rhat = torch.empty(P, dtype=torch.float64, device="cuda")
+    lib = _lib.load()
+    nbytes = int(lib.nax_diagnostics_workspace(C, S, P))  # 0: sizes the call below refuses
+    ws = torch.empty(nbytes + 256, dtype=torch.uint8, device="cuda")
     torch.cuda.synchronize()
-    _lib.check(_lib.load().nax_diagnostics(_lib.ptr(xf), C, S, P, _lib.ptr(ess), _lib.ptr(rhat)),
+    _lib.check(lib.nax_diagnostics_ws(_lib.ptr(xf), C, S, P, _lib.ptr(ess), _lib.ptr(rhat),
+                                      (ws.data_ptr() + 255) // 256 * 256, nbytes),
                "nax_diagnostics")
     return ess.reshape(rest), rhat.reshape(rest)
