@@ -561,6 +561,8 @@ def model_kernel_name(x_dtype, N, D, C, single=False):
     if x_dtype == "bf16":
         return f"logit_bf16_pipe<{dp}, {'true' if single else 'false'}>"
     if x_dtype == "fp8":
+        if C > 128:
+            return f"logit_split_kernel<{dp}, fp8>"
         return "logit_partial_f32<XFP8> (VALU tile, e4m3 decoded to fp32)"
     if C <= 16 and D <= 64 and N * D <= (1 << 20):
         return (f"persistent_kernel<LogisticChainModel<{32 if D <= 32 else 64}>> "
@@ -568,8 +570,8 @@ def model_kernel_name(x_dtype, N, D, C, single=False):
     if C < 32:
         return "logit_partial_f32 (VALU tile)"
     if C > 128:
-        return f"logit_mfma<FormF32,{dp}>"
-    return f"logit_partial_f32 or logit_mfma<FormF32,{dp}> (autotuned)"
+        return f"logit_split_kernel<{dp}, fp32>"
+    return f"logit_partial_f32 or logit_split_kernel<{dp}, fp32> (autotuned)"
 
 
 # HBM bytes per launch of the main kernel measured with rocprofv3 --pmc

@@ -30,7 +30,7 @@ extern "C" {
 
 #define NAX_X_F32 0
 #define NAX_X_BF16 1
-#define NAX_X_FP8 2 /* OCP e4m3fn + power-of-two column scales, VALU tile kernel */
+#define NAX_X_FP8 2 /* OCP e4m3fn + power-of-two column scales */
 
 typedef struct nax_sampler nax_sampler;
 
@@ -174,15 +174,18 @@ int nax_model_hier(nax_sampler* h, const float* d_x, const float* d_y, const int
 /* nax_model_logistic with the kernel choice for fp32 storage: 0 = auto
  * (one wavefront per chain in a persistent launch for <= 16 chains on
  * n*d <= 2^20, d <= 64; otherwise the VALU tile kernel or, from 32 chains
- * up, the fp32 MFMA kernel, whichever the autotuner times faster), 1 = VALU
- * tile kernel, 2 = fp32 MFMA, 3 = one wavefront per chain.  bf16 storage
+ * up, the matrix-core kernel, whichever the autotuner times faster), 1 = VALU
+ * tile kernel, 2 = matrix cores (X Z^T in fp32; X^T R by two fp16 terms per
+ * factor where rows and column ranges allow, else fp32), 3 = one wavefront per
+ * chain.  bf16 storage
  * always uses the matrix cores: 0 (auto) or 4 keep one bf16 copy of X and
  * read it transposed for X^T R with bf16 residuals; 2 keeps a second, fp16
  * copy for X^T R with fp16 residuals (twice the X bytes per evaluation, a
  * gradient rounding of 2^-11 instead of 2^-8 per term, and max|X| < 60000).
  * fp8 storage (NAX_X_FP8; the library quantises d_x as nax_fp8_quantize
- * does and keeps the codes) runs on the VALU tile kernel: 0 (auto, row
- * splits autotuned) or 1.  Other kernel values with bf16 or fp8 storage,
+ * does and keeps the codes): 0 (auto: the matrix cores for d <= 256 and
+ * n >= 65536, else the VALU tile kernel with autotuned row splits) or 1 (VALU
+ * tile kernel).  Other kernel values with bf16 or fp8 storage,
  * and 4 with fp32 storage, are refused (NAX_EINVAL). */
 int nax_model_logistic_ex(nax_sampler* h, const float* d_x, const float* d_y, int64_t n,
                           int32_t d, double prior_scale, int32_t x_dtype, int32_t kernel);

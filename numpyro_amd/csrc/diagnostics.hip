@@ -74,21 +74,6 @@ __host__ __device__ inline int diag_chain(int C, int g, int ng) {
 
 constexpr int kAggDoubles = 6;  // full and split (mean of means, m2 of means, sum of variances)
 
-// One 4-byte global->LDS load per lane (lane l writes LDS byte base + 4 l, base
-// wave-uniform in M0); the caller waits with vmcnt and a barrier.
-__device__ __forceinline__ void lds_dma4(const void* gptr, uint32_t base) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dword %0, off"
-      :
-      : "v"(gptr), "s"(base)
-      : "memory", "m0");
-}
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
 // Sums of NV values over the threads of a column (tid % PT), for every thread:
 // inside the wave by shuffles, then the waves' partials in wave order.
 template <int PT, int NV>

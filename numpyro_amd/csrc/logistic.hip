@@ -26,10 +26,6 @@
 
 namespace nax {
 
-__device__ __forceinline__ float softplusf_(float x) {
-  // max(x, 0) + log1p(exp(-|x|))  (distributions/util.py:317-320)
-  return fmaxf(x, 0.0f) + log1pf(__expf(-fabsf(x)));
-}
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
 // ---- X storage forms of the tile kernel ----------------------------------------
@@ -465,10 +461,15 @@ int fp8_quantize(const float* x, int64_t n, int d, uint8_t** q, float** scale, h
 }
 
 Potential* make_logistic_mfma(const float* x, const float* y, int64_t n, int d,
-                              double prior_scale, bool bf16, bool single, hipStream_t s,
+                              double prior_scale, bool single, hipStream_t s,
                               std::string* err);
 
-// fuse_variant: 0 = auto (matrix cores when num_chains >= 32), 1 = VALU tile
+int64_t logistic_split_min_rows();
+Potential* make_logistic_split(const float* x, const uint8_t* codes, const float* scales,
+                               const float* y, int64_t n, int d, double prior_scale,
+                               int num_chains, hipStream_t s, std::string* err);
+
+// fuse_variant: 0 = auto (fp32: matrix cores when num_chains >= 32), 1 = VALU tile
 // kernel, 2 = matrix cores, 3 = a group of wavefronts per chain.  bf16 always runs on
 // the matrix cores: 0 or 4 keep one X copy (bf16 residuals in X^T R), 2 keeps
 // a second, fp16 copy for X^T R with fp16 residuals.
@@ -480,14 +481,14 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
       *err = "bf16 storage takes kernel 0 or 4 (one copy of X) or 2 (two copies)";
       return nullptr;
     }
-    return make_logistic_mfma(x, y, n, d, prior_scale, true, fuse_variant != 2, s, err);
+    return make_logistic_mfma(x, y, n, d, prior_scale, fuse_variant != 2, s, err);
   }
   if (fuse_variant == 4) {
     *err = "kernel 4 (single-copy bf16) needs bf16 storage";
     return nullptr;
   }
   if (x_dtype == NAX_X_FP8 && fuse_variant != 0 && fuse_variant != 1) {
-    *err = "fp8 storage runs on the VALU tile kernel: kernel 0 (auto) or 1";
+    *err = "fp8 storage takes kernel 0 (auto) or 1 (the VALU tile kernel)";
     return nullptr;
   }
   if (x_dtype != NAX_X_F32 && x_dtype != NAX_X_FP8) {
@@ -500,10 +501,18 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
   if (!fp8 && (fuse_variant == 3 || (fuse_variant == 0 && num_chains <= 16 && d <= 64 &&
                                      (double)n * d <= (double)(1 << 20))))
     return make_logistic_chain(x, y, n, d, prior_scale, s, err);
-  const bool mfma = !fp8 && (fuse_variant == 2 ||
-                             (fuse_variant == 0 && num_chains >= 32 && d <= 256));
-  if (mfma && !(fuse_variant == 0 && num_chains <= 128 && d <= 320))
-    return make_logistic_mfma(x, y, n, d, prior_scale, false, false, s, err);
+  // fp8: the matrix cores from logistic_split_min_rows() rows on, for any number
+  // of chains (the tile kernel takes 8 chains at a time through a table lookup
+  // per element; a call at 500,000 x 250: 250 chains 15.0 ms against 1.0, 32 chains
+  // 2.24 against 0.68, 1 chain 0.94 against 0.62; 70,000 x 30, 2 chains 0.35 against
+  // 0.22)
+  const bool mfma = fp8 ? fuse_variant == 0 && d <= 256 && n >= logistic_split_min_rows()
+                        : fuse_variant == 2 || (fuse_variant == 0 && num_chains >= 32 && d <= 256);
+  auto matrix_form = [&](const uint8_t* codes, const float* scales) -> Potential* {
+    return make_logistic_split(x, codes, scales, y, n, d, prior_scale, num_chains, s, err);
+  };
+  if (mfma && !fp8 && !(fuse_variant == 0 && num_chains <= 128 && d <= 320))
+    return matrix_form(nullptr, nullptr);
   if (d > 320) {
     *err = "the fp32 logistic tile kernel supports dim <= 320";
     return nullptr;
@@ -523,10 +532,15 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
       delete p;
       return nullptr;
     }
+    if (mfma) {
+      Potential* q = matrix_form(p->q8, p->scale8);
+      delete p;
+      return q;
+    }
   }
   if (fuse_variant != 0 || num_chains < 1) return p;
   // Autotuner ("auto" kernel): row splits of the tile kernel, and for 32 <=
-  // C <= 128 the tile kernel against the fp32 MFMA kernel, each timed over a
+  // C <= 128 the tile kernel against the matrix-core kernel, each timed over a
   // few evaluations of all C chains at z = 0; the fastest is kept.
   const int C = num_chains;
   const int ld = (d + 63) / 64 * 64;
@@ -562,8 +576,7 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
     }
     p->rb_pick = best_rb;
     if (mfma) {
-      std::string e2;
-      Potential* q = make_logistic_mfma(x, y, n, d, prior_scale, false, false, s, &e2);
+      Potential* q = matrix_form(nullptr, nullptr);
       if (q) {
         if (time_it(q) < best_ms) best = q;
         else delete q;

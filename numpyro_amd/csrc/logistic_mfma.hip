@@ -1,4 +1,5 @@
-// Logistic potential + adjoint on the matrix cores (gfx950 MFMA), C chains.
+// Logistic potential + adjoint for bf16 designs on the matrix cores (gfx950
+// MFMA), C chains (fp32 and fp8 designs: logistic_split.hip).
 //
 // Same mathematics as logistic.hip (numpyro/distributions/discrete.py:244-263,
 // distributions/util.py:317-320, examples/covtype.py:66-71):
@@ -14,17 +15,15 @@
 // (c, h) must supply K-slots 8h..8h+7 of chain c: choosing the K order of
 // GEMM2 so that slot 8h + j of MFMA m is row 16m + 8(j/4) + 4h + j%4 makes that
 // operand exactly accumulator registers 8m..8m+7 -- R never leaves registers.
-// X is stored twice in fragment order (prepared once per model):
-//   A1[T][kk][lane][j] = X[32T + lane%32][KS kk + KS/2 (lane/32) + j]
-//   B2[T][m][dt][lane][j] = X[32T + row(m, lane/32, j)][32 dt + lane%32]
+// X is stored in fragment order (prepared once per model):
+//   A1[T][kk][lane][j] = X[32T + lane%32][16 kk + 8 (lane/32) + j]
+//   B2[T][m][dt][lane][j] = X[32T + row(m, lane/32, j)][32 dt + lane%32]  (two-copy form)
 // so every operand fetch is one coalesced load.  Blocks that walk the same
 // row tiles (same row split, different chain tiles) are placed on the same
 // XCD (blocks are dealt to the 8 XCDs round-robin) to share its L2.
 //
-// Precision forms:
-//   BF16: X in bf16 (RNE); Z enters as a bf16 hi+lo pair (two MFMAs), so the
-//         positions keep ~16 mantissa bits; R as bf16 hi+lo; fp32 accumulate.
-//   FP32: X, Z, R in fp32 on the fp32 MFMA (v_mfma_f32_32x32x2_f32).
+// Precision: X in bf16 (RNE); Z enters as a bf16 hi+lo pair (two MFMAs), so the
+// positions keep ~16 mantissa bits; fp32 accumulate.
 // Energies accumulate in fp64 per lane.  Partials per row split are summed in
 // a fixed order by logit_reduce (logistic.hip).
 #include <hip/hip_runtime.h>
@@ -42,26 +41,8 @@ namespace nax {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
-__device__ __forceinline__ float softplus_f(float x) {
-  return fmaxf(x, 0.0f) + log1pf(__expf(-fabsf(x)));
-}
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + __expf(-x)); }
-
-// r = sigmoid(l) - y and u = softplus(l) - y l (logistic_terms_f) with the
-// sign test shared: r = (l >= 0 ? 1 : e) / (1 + e) - y as one fma, and
-// max(l, 0) as a select on the same test.
-__device__ __forceinline__ void logit_terms(float l, float y, float& r, float& u) {
-  const bool pos = l >= 0.0f;
-  const float e = __builtin_amdgcn_exp2f(-fabsf(l) * 1.44269504088896341f);
-  const float d = 1.0f + e;
-  const float inv = __builtin_amdgcn_rcpf(d);
-  r = fmaf(pos ? 1.0f : e, inv, -y);
-  u = fmaf(__builtin_amdgcn_logf(d), 0.693147180559945309f, fmaf(-y, l, pos ? l : 0.0f));
-}
-
-
 // ---- fragment-order preparation -------------------------------------------------
-// KS = K per MFMA (16 for bf16, 2 for fp32); Dp = D rounded up to 32.
+// KS = K per MFMA; Dp = D rounded up to 32.
 // SWZ (single-copy bf16 form): within each 64-fragment block the second
 // half's rows are stored XOR 4 (position p holds lane p ^ 4 for p >= 32), so
 // the transposed GEMM2 reads of a row's two 8-column halves fall on
@@ -121,250 +102,10 @@ __global__ void pad_y(const float* __restrict__ y, int64_t N, int64_t Np, float*
     out[i] = i < N ? y[i] : 0.5f;
 }
 
-// ---- the fused kernel ----------------------------------------------------------------
-struct FormBF16 {
-  static constexpr int KS = 16;
-  typedef bf16x8 frag;
-  static __device__ __forceinline__ f32x16 mma(frag a, frag b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-};
-struct FormF32 {
-  static constexpr int KS = 2;
-  typedef float frag;
-  static __device__ __forceinline__ f32x16 mma(frag a, frag b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-};
-
-template <typename F, int DP>
-__global__ void __launch_bounds__(256, 1)
-logit_mfma(const typename F::frag* __restrict__ A1, const typename F::frag* __restrict__ B2,
-           const float* __restrict__ ypad, int64_t N, int64_t ntile, const float* __restrict__ Z,
-           int ldz, int D, int C, float* __restrict__ wsg,
-           double* __restrict__ wsu, const int* __restrict__ act, const int* __restrict__ nact) {
-  constexpr int KS = F::KS;
-  constexpr int KK = DP / KS;   // GEMM1 K steps
-  constexpr int DT = DP / 32;   // GEMM2 d tiles
-  constexpr int M2 = 32 / KS;   // GEMM2 MFMAs per d tile and row tile
-  constexpr bool BF = (KS == 16);
-  typedef typename F::frag frag;
-  // one row tile in LDS: A1 part, B2 part, 32 labels
-  constexpr int ABYTES = KK * 64 * (int)sizeof(frag);
-  constexpr int BBYTES = M2 * DT * 64 * (int)sizeof(frag);
-  constexpr int TBYTES = ABYTES + BBYTES + 128;
-  constexpr int PF = (ABYTES + BBYTES) / (256 * 16);   // 16-byte chunks per thread
-  constexpr int PA = ABYTES / 16;                      // chunks in the A1 part
-  static_assert((ABYTES + BBYTES) % (256 * 16) == 0, "tile must split into 16-byte chunks");
-  __shared__ __attribute__((aligned(16))) char lds[2][TBYTES];
-
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int l = tid & 63;
-  const int cl = l & 31, h = l >> 5;
-  // XCD-aware block placement: blocks of one row split share an XCD.
-  // Chains are taken through the compacted list act[0..*nact) of the chains
-  // that requested a gradient (all C in order when act is null); column
-  // index ci addresses the workspaces (row stride CT * 128), chain act[ci]
-  // the positions.  The chain tiles and row splits are laid out for the
-  // requesting chains only, over the whole launch.
-  const int n_act = act ? *nact : C;
-  if (n_act <= 0) return;
-  int CT, RB;
-  logit_split(n_act, (int)gridDim.x, ntile, CT, RB);
-  const int ldw = CT * 128;
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7;
-  const int slot = bid >> 3;
-  const int ct = slot % CT;
-  const int rb = (slot / CT) * 8 + xcd;
-  if (rb >= RB) return;  // uniform over the block
-  const int c0 = ct * 128 + wave * 32;
-  const bool cvalid = c0 + cl < n_act;
-  const int c = cvalid ? (act ? act[c0 + cl] : c0 + cl) : 0;
-
-  // Z fragments (B operand of GEMM1): lane (c, h) holds Z[c][KS kk + KS/2 h + j]
-  frag zh[KK];
-  frag zlo[BF ? KK : 1];
-#pragma unroll
-  for (int kk = 0; kk < KK; ++kk) {
-    if constexpr (BF) {
-      bf16x8 hi, lo;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        int d = 16 * kk + 8 * h + j;
-        float v = (cvalid && d < D) ? Z[(size_t)c * ldz + d] : 0.0f;
-        __bf16 b = (__bf16)v;
-        hi[j] = b;
-        lo[j] = (__bf16)(v - (float)b);
-      }
-      zh[kk] = hi;
-      zlo[kk] = lo;
-    } else {
-      int d = 2 * kk + h;
-      zh[kk] = (cvalid && d < D) ? Z[(size_t)c * ldz + d] : 0.0f;
-    }
-  }
-
-  f32x16 g[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) g[dt][v] = 0.0f;
-  CompSum u;  // fp64 energy over this lane's tiles, compensated
-
-  // ---- tile staging: global -> registers (prefetch) -> LDS ----
-  // Clang vector types, not HIP's uint4/float4 structs: an array of those
-  // stays in scratch memory, and every prefetch then waits for its loads.
-  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  u32x4 pf[PF];
-  f32x4 pfy;
-  auto load_tile = [&](int64_t t) {
-    const u32x4* ga = (const u32x4*)(A1 + (size_t)t * KK * 64);
-    const u32x4* gb = (const u32x4*)(B2 + (size_t)t * M2 * DT * 64);
-#pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int idx = tid + 256 * p;
-      if constexpr (PA % 256 == 0) {  // the source of chunk p is known at compile time
-        if (p < PA / 256) pf[p] = ga[idx];
-        else pf[p] = gb[idx - PA];
-      } else {
-        pf[p] = idx < PA ? ga[idx] : gb[idx - PA];
-      }
-    }
-    pfy = ((const f32x4*)(ypad + 32 * t))[tid & 7];
-  };
-  auto store_tile = [&](int buf) {
-    u32x4* s4 = (u32x4*)lds[buf];
-#pragma unroll
-    for (int p = 0; p < PF; ++p) s4[tid + 256 * p] = pf[p];
-    // every thread stores its copy of label chunk tid & 7 (equal values):
-    // an unconditional store keeps the label load at the top of the tile
-    ((f32x4*)(lds[buf] + ABYTES + BBYTES))[tid & 7] = pfy;
-  };
-
-  int64_t t = rb;
-  int cur = 0;
-  if (t < ntile) {
-    load_tile(t);
-    store_tile(0);
-  }
-  __syncthreads();
-  for (; t < ntile; t += RB) {
-    const bool has_next = t + RB < ntile;
-    // unconditional (the last tile reloads itself, unused), so that the
-    // prefetch registers are written on every path and stay registers
-    load_tile(has_next ? t + RB : t);
-    // keep the prefetch loads here: left to itself the scheduler sinks them
-    // next to their LDS stores at the end of the tile and waits on them
-    __builtin_amdgcn_sched_barrier(0);
-    const frag* la = (const frag*)lds[cur];
-    const frag* lb = (const frag*)(lds[cur] + ABYTES);
-    const float* ly = (const float*)(lds[cur] + ABYTES + BBYTES);
-
-    // GEMM1: L = X_tile Z^T
-    f32x16 L;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) L[v] = 0.0f;
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      frag af = la[kk * 64 + l];
-      L = F::mma(af, zh[kk], L);
-      if constexpr (BF) L = F::mma(af, zlo[kk], L);
-    }
-    // epilogue: register v holds row 8(v/4) + 4h + v%4 (padded rows give
-    // r = 0 and u = fp32(ln 2), removed by the reduction)
-    float rv[16];
-    float us = 0.0f;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float4 yq = *(const float4*)(ly + 8 * q + 4 * h);
-      const float yy[4] = {yq.x, yq.y, yq.z, yq.w};
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        float uu;
-        logit_terms(L[4 * q + m], yy[m], rv[4 * q + m], uu);
-        us += uu;
-      }
-    }
-    u.add((double)us);
-    // GEMM2: G^T += R^T X_tile
-    if constexpr (BF) {
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        bf16x8 rh, rl;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          __bf16 hb = (__bf16)rv[8 * m + j];
-          rh[j] = hb;
-          rl[j] = (__bf16)(rv[8 * m + j] - (float)hb);
-        }
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          frag bf = lb[(m * DT + dt) * 64 + l];
-          g[dt] = F::mma(rh, bf, g[dt]);
-          g[dt] = F::mma(rl, bf, g[dt]);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int m = 0; m < 16; ++m) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          frag bf = lb[(m * DT + dt) * 64 + l];
-          g[dt] = F::mma(rv[m], bf, g[dt]);
-        }
-      }
-    }
-    store_tile(cur ^ 1);  // unconditional: the other buffer is not read after the last tile
-    __syncthreads();
-    cur ^= 1;
-  }
-
-  // G^T partial: register v of tile dt is chain 8(v/4) + 4h + v%4 (relative
-  // to c0), column d = 32 dt + cl.
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
-    const int d = 32 * dt + cl;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int ci = c0 + 8 * (v / 4) + 4 * h + (v % 4);
-      if (ci < n_act && d < D) wsg[((size_t)rb * ldw + ci) * D + d] = g[dt][v];
-    }
-  }
-  CompSum uo;
-  uo.s = __shfl_xor(u.s, 32, 64);
-  uo.c = __shfl_xor(u.c, 32, 64);
-  u.add(uo);
-  const double ut = u.value();
-  if (h == 0 && cvalid) wsu[(size_t)rb * ldw + c0 + cl] = ut;
-}
-
 // ---- pipelined BF16 kernel --------------------------------------------------------
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 
-// One 16-byte global->LDS load per lane (global_load_lds_dwordx4): lane l
-// writes LDS byte lds_base + 16 l (lds_base wave-uniform, in M0).  Issued as
-// inline assembly so that the compiler does not tie later LDS reads to it:
-// given the builtin, the waitcnt pass makes every later ds_read of the block
-// wait for all outstanding LDS-DMA loads (vmcnt(0)), which turns a prefetch
-// several tiles ahead into a wait on the tile just issued.  The kernel waits
-// for these loads itself with counted s_waitcnt vmcnt + a barrier.
-__device__ __forceinline__ void lds_dma16(const void* gptr, uint32_t lds_base) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
-      :
-      : "v"(gptr), "s"(lds_base)
-      : "memory", "m0");
-}
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
-// Software-pipelined form of logit_mfma for bf16 X.  The block's row tiles
+// The software-pipelined kernel.  The block's row tiles
 // i = 0..n-1 (tile rb + i RB) stream through LDS by direct global->LDS loads
 // (no staging registers).  Iteration i runs, as one branch-free basic block,
 // the epilogue of tile i (VALU) interleaved in source order with GEMM1 of
@@ -748,8 +489,7 @@ struct LogisticMfma : Potential {
   int64_t n = 0, ntile = 0;
   int d = 0, dp = 0;
   double prior_scale = 1.0;
-  bool bf16 = true;
-  bool single = false;  // bf16 only: one X copy, GEMM2 transposed from it, bf16 R
+  bool single = false;  // one X copy, GEMM2 transposed from it, bf16 R
   void* a1 = nullptr;
   void* b2 = nullptr;
   float* ypad = nullptr;
@@ -763,16 +503,15 @@ struct LogisticMfma : Potential {
   }
   int dim() const override { return d; }
   const char* name() const override {
-    return bf16 ? (single ? "logit_mfma_bf16_single" : "logit_mfma_bf16") : "logit_mfma_f32";
+    return single ? "logit_mfma_bf16_single" : "logit_mfma_bf16";
   }
   double alg_flops(int C) const override { return 4.0 * (double)n * d * C; }
-  double alg_bytes(int C) const override { return (bf16 ? 2.0 : 4.0) * (double)n * d + 4.0 * n; }
+  double alg_bytes(int C) const override { return 2.0 * (double)n * d + 4.0 * n; }
 
   hipError_t setup(const float* x, const float* y, hipStream_t s) {
     ntile = (n + 31) / 32;
     dp = (d + 31) / 32 * 32;
-    const size_t elt = bf16 ? 2 : 4;
-    const size_t per = (size_t)ntile * 32 * dp * elt;
+    const size_t per = (size_t)ntile * 32 * dp * 2;
     hipError_t e = hipMalloc(&a1, per);
     if (e != hipSuccess) return e;
     if (!single) {
@@ -786,9 +525,9 @@ struct LogisticMfma : Potential {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, dev) == hipSuccess) num_cu = prop.multiProcessorCount;
     const int blocks = 4096;
-    if (bf16 && single) {
+    if (single) {
       hipLaunchKernelGGL((prep_a1<__bf16, 16, true>), dim3(blocks), dim3(256), 0, s, x, n, d, dp, ntile, (__bf16*)a1);
-    } else if (bf16) {
+    } else {
       unsigned* dmax = nullptr;
       e = hipMallocAsync((void**)&dmax, sizeof(unsigned), s);
       if (e != hipSuccess) return e;
@@ -804,9 +543,6 @@ struct LogisticMfma : Potential {
       if (!(fmax_x < 60000.0f)) return hipErrorInvalidValue;  // fp16 GEMM2 range
       hipLaunchKernelGGL((prep_a1<__bf16, 16>), dim3(blocks), dim3(256), 0, s, x, n, d, dp, ntile, (__bf16*)a1);
       hipLaunchKernelGGL((prep_b2<_Float16, 16, true>), dim3(blocks), dim3(256), 0, s, x, n, d, dp, ntile, (_Float16*)b2);
-    } else {
-      hipLaunchKernelGGL((prep_a1<float, 2>), dim3(blocks), dim3(256), 0, s, x, n, d, dp, ntile, (float*)a1);
-      hipLaunchKernelGGL((prep_b2<float, 2>), dim3(blocks), dim3(256), 0, s, x, n, d, dp, ntile, (float*)b2);
     }
     hipLaunchKernelGGL(pad_y, dim3(1024), dim3(256), 0, s, y, n, ntile * 32, ypad);
     e = hipGetLastError();
@@ -842,22 +578,6 @@ struct LogisticMfma : Potential {
       ws_elems = need;
     }
     mark_begin(s);
-#define NAX_L(FORM, DPV)                                                                      \
-  hipLaunchKernelGGL((logit_mfma<FORM, DPV>), dim3(nblk), dim3(256), 0, s,                    \
-                     (const FORM::frag*)a1, (const FORM::frag*)b2, ypad, n, ntile, z, ldz, d, C, \
-                     wsg, wsu, act, nact)
-#define NAX_DP(FORM)                    \
-  switch (dp) {                         \
-    case 32: NAX_L(FORM, 32); break;    \
-    case 64: NAX_L(FORM, 64); break;    \
-    case 96: NAX_L(FORM, 96); break;    \
-    case 128: NAX_L(FORM, 128); break;  \
-    case 160: NAX_L(FORM, 160); break;  \
-    case 192: NAX_L(FORM, 192); break;  \
-    case 224: NAX_L(FORM, 224); break;  \
-    case 256: NAX_L(FORM, 256); break;  \
-    default: return hipErrorInvalidValue; \
-  }
 #define NAX_P(DPV, SGL)                                                                        \
   hipLaunchKernelGGL((logit_bf16_pipe<DPV, SGL>), dim3(nblk), dim3(256), 0, s,                 \
                      (const bf16x8*)a1, (const f16x8*)b2, ypad, n, ntile, z, ldz, d, C, wsg,   \
@@ -874,17 +594,13 @@ struct LogisticMfma : Potential {
     case 256: NAX_P(256, SGL); break;       \
     default: return hipErrorInvalidValue;   \
   }
-    if (bf16 && single) {
+    if (single) {
       NAX_PDP(true)
-    } else if (bf16) {
-      NAX_PDP(false)
     } else {
-      NAX_DP(FormF32)
+      NAX_PDP(false)
     }
 #undef NAX_PDP
 #undef NAX_P
-#undef NAX_DP
-#undef NAX_L
     mark_end(s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -899,7 +615,7 @@ struct LogisticMfma : Potential {
 };
 
 Potential* make_logistic_mfma(const float* x, const float* y, int64_t n, int d,
-                              double prior_scale, bool bf16, bool single, hipStream_t s,
+                              double prior_scale, bool single, hipStream_t s,
                               std::string* err) {
   if (d > 256) {
     *err = "the MFMA logistic kernels support dim <= 256";
@@ -909,12 +625,11 @@ Potential* make_logistic_mfma(const float* x, const float* y, int64_t n, int d,
   p->n = n;
   p->d = d;
   p->prior_scale = prior_scale;
-  p->bf16 = bf16;
-  p->single = bf16 && single;
+  p->single = single;
   hipError_t e = p->setup(x, y, s);
   if (e != hipSuccess) {
-    *err = std::string("logistic MFMA setup: ") + hipGetErrorString(e) +
-           (bf16 && !single && e == hipErrorInvalidValue
+    *err = std::string("logistic bf16 setup: ") + hipGetErrorString(e) +
+           (!single && e == hipErrorInvalidValue
                 ? " (the two-copy bf16 form needs max|X| < 60000)" : "");
     delete p;
     return nullptr;

@@ -285,4 +285,80 @@ __device__ __forceinline__ void logistic_terms_f(float l, float y, float& r, flo
   u = fmaf(__builtin_amdgcn_logf(d), 0.693147180559945309f, fmaxf(l, 0.0f) - y * l);
 }
 
+// r = sigmoid(l) - y and u = softplus(l) - y l (logistic_terms_f) with the
+// sign test shared: r = (l >= 0 ? 1 : e) / (1 + e) - y as one fma, and
+// max(l, 0) as a select on the same test.
+__device__ __forceinline__ void logit_terms(float l, float y, float& r, float& u) {
+  const bool pos = l >= 0.0f;
+  const float e = __builtin_amdgcn_exp2f(-fabsf(l) * 1.44269504088896341f);
+  const float d = 1.0f + e;
+  const float inv = __builtin_amdgcn_rcpf(d);
+  r = fmaf(pos ? 1.0f : e, inv, -y);
+  u = fmaf(__builtin_amdgcn_logf(d), 0.693147180559945309f, fmaf(-y, l, pos ? l : 0.0f));
+}
+
+// max(x, 0) + log1p(exp(-|x|))  (distributions/util.py:317-320)
+__device__ __forceinline__ float softplusf_(float x) {
+  return fmaxf(x, 0.0f) + log1pf(__expf(-fabsf(x)));
+}
+
+// log1p(e) for e in [0, 1], as 2 atanh(s) with s = e / (2 + e) <= 1/3: the
+// odd series up to s^17 (next term 2e-9), every step rounded to nearest.
+// A quarter of log1pf's instructions.
+__device__ __forceinline__ float log1p_unit(float e) {
+  const float den = 2.0f + e;
+  const float inv = __builtin_amdgcn_rcpf(den);
+  const float s0 = e * inv;
+  const float s = fmaf(fmaf(-s0, den, e), inv, s0);
+  const float t = s * s;
+  float p = 1.0f / 17.0f;
+  p = fmaf(p, t, 1.0f / 15.0f);
+  p = fmaf(p, t, 1.0f / 13.0f);
+  p = fmaf(p, t, 1.0f / 11.0f);
+  p = fmaf(p, t, 1.0f / 9.0f);
+  p = fmaf(p, t, 1.0f / 7.0f);
+  p = fmaf(p, t, 1.0f / 5.0f);
+  p = fmaf(p, t, 1.0f / 3.0f);
+  const float s2 = s + s;
+  return fmaf(s2 * t, p, s2);
+}
+
+// The terms with log1p (exact for small e, where log2(1 + e) has lost e's low
+// bits, as the VALU tile kernel has them), r as above.
+__device__ __forceinline__ void logit_terms_log1p(float l, float y, float& r, float& u) {
+  const float e = __expf(-fabsf(l));
+  r = fmaf(l >= 0.0f ? 1.0f : e, __builtin_amdgcn_rcpf(1.0f + e), -y);
+  u = fmaf(-y, l, fmaxf(l, 0.0f) + log1p_unit(e));
+}
+
+// One 16-byte global->LDS load per lane (global_load_lds_dwordx4): lane l
+// writes LDS byte lds_base + 16 l (lds_base wave-uniform, in M0).  Issued as
+// inline assembly so that the compiler does not tie later LDS reads to it:
+// given the builtin, the waitcnt pass makes every later ds_read of the block
+// wait for all outstanding LDS-DMA loads (vmcnt(0)), which turns a prefetch
+// several tiles ahead into a wait on the tile just issued.  The kernel waits
+// for these loads itself with counted s_waitcnt vmcnt + a barrier.
+__device__ __forceinline__ void lds_dma16(const void* gptr, uint32_t lds_base) {
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, off"
+      :
+      : "v"(gptr), "s"(lds_base)
+      : "memory", "m0");
+}
+// The same with 4 bytes per lane (lane l writes LDS byte lds_base + 4 l).
+__device__ __forceinline__ void lds_dma4(const void* gptr, uint32_t lds_base) {
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %0, off"
+      :
+      : "v"(gptr), "s"(lds_base)
+      : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
 }  // namespace nax

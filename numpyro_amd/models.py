@@ -92,11 +92,11 @@ class LogisticRegression(Model):
     ``"bf16"`` (MFMA; by default one bf16 copy of X with bf16 residuals in
     X^T R, ``kernel="two-copy"`` adds an fp16 copy for fp16 residuals) or
     ``"fp8"`` (OCP e4m3fn bytes with a power-of-two scale per column, decoded
-    exactly in the VALU tile kernel, fp32 arithmetic; the quantised design
-    defines the model).  The fp8 MFMA is not used: both of its operands are
-    8-bit, so the positions would need a three-term e4m3 split (as costly as
-    the two bf16 products) and the residuals of X^T R would keep 3 mantissa
-    bits."""
+    exactly, X B in fp32 arithmetic; the quantised design defines the model;
+    ``kernel="tile"`` keeps it off the matrix cores).  The fp8 MFMA is not
+    used: both of its operands are 8-bit, so the positions would need a
+    three-term e4m3 split (as costly as the two bf16 products) and the
+    residuals of X^T R would keep 3 mantissa bits."""
 
     def __init__(self, X, y, prior_scale=1.0, x_dtype="fp32", kernel="auto"):
         X = torch.as_tensor(X)
@@ -120,7 +120,7 @@ class LogisticRegression(Model):
             raise ValueError("bf16 storage runs on the matrix cores: kernel 'auto', 'single' "
                              "or 'two-copy'")
         if _canon(x_dtype) == "fp8" and kernel not in ("auto", "tile"):
-            raise ValueError("fp8 storage runs on the VALU tile kernel: kernel 'auto' or 'tile'")
+            raise ValueError("fp8 storage takes kernel 'auto' or 'tile' (the VALU tile kernel)")
         self.kernel = kernel
         self.site_sizes = (("coefs", self.dim, None),)
 
