@@ -320,6 +320,15 @@ int nax_logistic_potential_grad_noalloc(const float* d_x, const float* d_y, int6
 int nax_potential_grad(nax_sampler* h, const float* d_z, int32_t ld, int32_t count,
                        double* d_pe, float* d_grad);
 
+/* The same enqueued on the caller's stream (a hipStream_t; NULL = the null
+ * stream) without waiting for it: pe and grad are written in stream order.
+ * Calls on several streams or threads are ordered behind one another (they
+ * share the model's workspaces), and so are the sampler's own calls behind
+ * them; none may run beside nax_run on the same sampler.  A subsampled model's
+ * indices must not be under update (nax_ecs_gibbs) when it is called. */
+int nax_potential_grad_on(nax_sampler* h, const float* d_z, int32_t ld, int32_t count,
+                          double* d_pe, float* d_grad, void* stream);
+
 /* L velocity_verlet steps (hmc_util.py:262-311) for C chains in place:
  * d_z, d_r, d_grad [C, dim]; d_pe [C]; d_inverse_mass_matrix [dim]. */
 int nax_leapfrog(nax_sampler* h, float* d_z, float* d_r, float* d_grad, double* d_pe,

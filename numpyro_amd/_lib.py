@@ -99,6 +99,8 @@ SIGNATURES = {
     "nax_set_adapt_state": (C.c_int, [C.c_void_p, C.POINTER(nax_adapt_view)]),
     "nax_potential_grad": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32,
                                      C.c_void_p, C.c_void_p]),
+    "nax_potential_grad_on": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32,
+                                        C.c_void_p, C.c_void_p, C.c_void_p]),
     "nax_logistic_potential_grad_noalloc": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int64,
                                                       C.c_int32, C.c_double, C.c_void_p,
                                                       C.c_int32, C.c_int32, C.c_void_p,

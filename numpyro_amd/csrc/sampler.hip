@@ -268,6 +268,13 @@ struct nax_sampler {
   double timing_ms = 0.0;
   int64_t timing_n = 0;
   std::vector<hipEvent_t> ev;
+  // nax_potential_grad_on: recorded behind the last evaluation on a caller's
+  // stream; whatever uses the model's workspaces next on another stream waits
+  // for it
+  std::mutex on_mu;
+  hipEvent_t on_done = nullptr;
+  hipStream_t on_stream = nullptr;
+  bool on_pending = false;
 };
 
 static const int kBatch = 16;
@@ -282,6 +289,14 @@ static const int kBatch = 16;
   } while (0)
 
 extern "C" const char* nax_last_error(void) { return g_err.c_str(); }
+
+// Orders the sampler's own stream behind evaluations on callers' streams.
+static hipError_t wait_callers(nax_sampler* h) {
+  std::lock_guard<std::mutex> lk(h->on_mu);
+  if (!h->on_pending) return hipSuccess;
+  h->on_pending = false;
+  return hipStreamWaitEvent(h->stream, h->on_done, 0);
+}
 
 static std::vector<int> schedule_ends(int num_steps) {
   // build_adaptation_schedule (numpyro/infer/hmc_util.py:387-436)
@@ -391,6 +406,10 @@ extern "C" int nax_create(const nax_config* c, nax_sampler** out) {
 extern "C" void nax_destroy(nax_sampler* h) {
   if (!h) return;
   if (h->stream) hipStreamSynchronize(h->stream);
+  if (h->on_done) {
+    (void)hipEventSynchronize(h->on_done);
+    (void)hipEventDestroy(h->on_done);
+  }
   delete h->pot;
   hipFree(h->vec); hipFree(h->wel); hipFree(h->st); hipFree(h->zreq); hipFree(h->gout);
   hipFree(h->peout); hipFree(h->ctr); hipFree(h->gevals); hipFree(h->active);
@@ -496,6 +515,7 @@ extern "C" int nax_ecs_gibbs(nax_sampler* h, float* accept_prob) {
   if (!h->initialized) { set_error("nax_ecs_gibbs before nax_init"); return NAX_ESTATE; }
   if (!h->pot) { set_error("nax_ecs_gibbs: no subsampled model set"); return NAX_ESTATE; }
   const EngineCfg& e = h->cfg;
+  NAX_HIP(wait_callers(h));
   hipError_t r = h->pot->ecs_gibbs(h->stream, h->st, h->vec + (size_t)V_Z * e.Dp,
                                    h->vec + (size_t)V_G * e.Dp, e.nvec * e.Dp, accept_prob);
   if (r == hipErrorNotSupported) {
@@ -634,6 +654,7 @@ extern "C" int nax_init(nax_sampler* h, const float* z0, const uint32_t* keys,
   if (!h || !z0 || !keys) { set_error("nax_init: null argument"); return NAX_EINVAL; }
   if (!h->pot && !h->external) { set_error("nax_init: no model set"); return NAX_ESTATE; }
   const EngineCfg& e = h->cfg;
+  NAX_HIP(wait_callers(h));
   uint32_t* dkeys = nullptr;
   NAX_HIP(hipMallocAsync((void**)&dkeys, sizeof(uint32_t) * 2 * e.C, h->stream));
   NAX_HIP(hipMemcpyAsync(dkeys, keys, sizeof(uint32_t) * 2 * e.C, hipMemcpyHostToDevice, h->stream));
@@ -675,6 +696,7 @@ extern "C" int nax_run(nax_sampler* h, int64_t target, const nax_collect* c, int
   if (!h->initialized) { set_error("nax_run before nax_init"); return NAX_ESTATE; }
   if (h->external || !h->pot) { set_error("nax_run needs a built-in model; use nax_advance"); return NAX_ESTATE; }
   Collect col = to_collect(c);
+  NAX_HIP(wait_callers(h));
   NAX_HIP(hipMemsetAsync(h->gevals, 0, sizeof(int64_t), h->stream));
   if (h->pot->persistent()) {
     // Whole loop on the device, in chunks of iterations with progress
@@ -1011,8 +1033,30 @@ extern "C" int nax_potential_grad(nax_sampler* h, const float* z, int32_t ld, in
   if (!h || !z || !pe || !g) { set_error("null argument"); return NAX_EINVAL; }
   if (!h->pot) { set_error("no built-in model set"); return NAX_ESTATE; }
   if (count <= 0 || ld < h->cfg.D) { set_error("bad count / ld"); return NAX_EINVAL; }
+  NAX_HIP(wait_callers(h));
   NAX_HIP(h->pot->eval(h->stream, z, ld, count, pe, g, ld));
   NAX_HIP(hipStreamSynchronize(h->stream));
+  return NAX_OK;
+}
+
+// On the caller's stream there is nothing to wait for on the host: a call with
+// a small model is a few launches (potential_energy and its gradient, 4 chains,
+// 1000 x 26: 180 us with the waits, padding copies and clears of the synchronous
+// call around it, 100 without).
+extern "C" int nax_potential_grad_on(nax_sampler* h, const float* z, int32_t ld, int32_t count,
+                                     double* pe, float* g, void* stream) {
+  if (!h || !z || !pe || !g) { set_error("null argument"); return NAX_EINVAL; }
+  if (!h->pot) { set_error("no built-in model set"); return NAX_ESTATE; }
+  if (count <= 0 || ld < h->cfg.D) { set_error("bad count / ld"); return NAX_EINVAL; }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  std::lock_guard<std::mutex> lk(h->on_mu);
+  if (!h->on_done)
+    NAX_HIP(hipEventCreateWithFlags(&h->on_done, hipEventDisableTiming));
+  if (h->on_pending && h->on_stream != s) NAX_HIP(hipStreamWaitEvent(s, h->on_done, 0));
+  NAX_HIP(h->pot->eval(s, z, ld, count, pe, g, ld));
+  NAX_HIP(hipEventRecord(h->on_done, s));
+  h->on_stream = s;
+  h->on_pending = true;
   return NAX_OK;
 }
 
@@ -1021,6 +1065,7 @@ extern "C" int nax_leapfrog(nax_sampler* h, float* z, float* r, float* g, double
   if (!h || !z || !r || !g || !pe || !imm) { set_error("null argument"); return NAX_EINVAL; }
   if (!h->pot) { set_error("no built-in model set"); return NAX_ESTATE; }
   const EngineCfg& e = h->cfg;
+  NAX_HIP(wait_callers(h));
   dim3 grid((e.D + 127) / 128, e.C);
   for (int s = 0; s < L; ++s) {
     hipLaunchKernelGGL(lf_half_kernel, grid, dim3(128), 0, h->stream, e.C, e.D, e.D, z, r, g,

@@ -362,15 +362,22 @@ def _device_value_and_grad(model, z):
     eng = cache.get(C)
     if eng is None:
         eng = cache[C] = Engine(model, C, "NUTS", 0)
-    ld = _lib.stride(eng.h)
-    zp = torch.zeros((C, ld), dtype=torch.float32, device="cuda")
-    zp[:, :model.dim] = z.detach().to(device="cuda", dtype=torch.float32)
+    if torch.cuda.is_current_stream_capturing():
+        # a graph would keep the addresses of the model's workspaces
+        raise RuntimeError("potential_energy cannot be captured in a graph (see "
+                           "nax_logistic_potential_grad_noalloc)")
+    D = model.dim
+    zp = z.detach().to(device="cuda", dtype=torch.float32).contiguous()
     pe = torch.empty(C, dtype=torch.float64, device="cuda")
-    g = torch.zeros((C, ld), dtype=torch.float32, device="cuda")
-    torch.cuda.synchronize()
-    _lib.check(_lib.load().nax_potential_grad(eng.h, _lib.ptr(zp), ld, C, _lib.ptr(pe),
-                                              _lib.ptr(g)), "nax_potential_grad")
-    return pe, g[:, :model.dim].contiguous()
+    # ragged models leave the entries past a chain's own size alone
+    g = (torch.empty if model.site_sizes else torch.zeros)((C, D), dtype=torch.float32,
+                                                           device="cuda")
+    stream = torch.cuda.current_stream()
+    zp.record_stream(stream)  # a caller's z may come from another stream's memory
+    _lib.check(_lib.load().nax_potential_grad_on(eng.h, _lib.ptr(zp), D, C, _lib.ptr(pe),
+                                                 _lib.ptr(g), stream.cuda_stream),
+               "nax_potential_grad")
+    return pe, g
 
 
 class _PotentialEnergy(torch.autograd.Function):
