@@ -196,15 +196,17 @@ logit_partial_f32(XL X, const float* __restrict__ y, int64_t N, int D,
 }
 
 // Sums the row-split partials and adds the Normal(0, s) prior; block ci
-// reduces workspace column ci.  Gradient: with D <= 128 the 256 threads form
-// 256 / DP2 groups (DP2 = D rounded up to a power of two), thread (group q,
-// column d) adds the splits q, q + groups, ... in order and the group sums
-// are added in group order; wider rows take a column per thread.  Energy:
-// thread t adds the splits t, t + 256, ... into a compensated sum and the
-// 256 sums are combined in a fixed pairwise tree.  Every order is fixed, so
-// results repeat bit for bit; the splits are read by all threads at once
-// instead of one column's (or, for the energy, one thread's) dependent loop.
-__global__ void __launch_bounds__(256)
+// reduces workspace column ci.  Gradient: with dp = D rounded up to 64 the
+// block's NT threads form NT / dp groups; thread (group q, column d) adds the
+// splits q, q + groups, ... in order, eight loads in flight, and the group sums
+// are added in group order.  Energy: thread t adds the splits t, t + NT, ... into a
+// compensated sum and the threads' sums are combined in a fixed pairwise tree.
+// Every order is fixed, so results repeat bit for bit.
+// Bound: the latency of a column's loads, so NT is 1024 while the chains' blocks
+// leave the chip room (256 threads before: 2048 splits of 1 chain x 55 32.8 -> 5.8
+// us, 256 of 256 x 55 20.4 -> 7.6, 128 of 250 x 250 35.0 -> 9.0), and 256 beyond 512
+// chains (32 splits of 1024 x 256: 13.3 us, 14.6 with 1024 threads).
+__global__ void __launch_bounds__(kReduceThreads)
 logit_reduce(const float* __restrict__ wsg, const double* __restrict__ wsu, int RB, int C,
              int D, const float* __restrict__ Z, int ldz, double inv_s2, double log_norm,
              double u_offset, double* __restrict__ pe, float* __restrict__ g, int ldg,
@@ -225,60 +227,61 @@ logit_reduce(const float* __restrict__ wsg, const double* __restrict__ wsu, int 
     ldw = CT * 128;
   }
   const int t = threadIdx.x;
-  __shared__ double red[256];
-  __shared__ double us[256], uc[256];
-  __shared__ float gred[256];
-  int dp2 = 1;
-  while (dp2 < D) dp2 <<= 1;
+  const int lane = t & (NAX_WAVE - 1), wave = t / NAX_WAVE;
+  const int NT = blockDim.x, NW = NT / NAX_WAVE;
+  constexpr int kWaves = kReduceThreads / NAX_WAVE;
+  __shared__ float gred[kReduceThreads];
+  __shared__ double us[kWaves], uc[kWaves], pw[kWaves];
+  const int dp = (D + NAX_WAVE - 1) / NAX_WAVE * NAX_WAVE;
+  const int ng = max(1, NT / dp), q = dp < NT ? t / dp : 0, d0 = dp < NT ? t % dp : t;
   double pr = 0.0;
-  if (dp2 <= 128) {
-    const int ng = 256 / dp2, q = t / dp2, d = t % dp2;
+  for (int b = 0; b < D; b += NT) {  // one round unless D > NT
+    const int d = b + d0;
     float sg = 0.0f;
-    if (d < D)
-      for (int r = q; r < RB; r += ng) sg += wsg[((size_t)r * ldw + ci) * D + d];
+    if (q < ng && d < D) {
+      const float* p = wsg + (size_t)ci * D + d;
+      const size_t st = (size_t)ldw * D;
+#pragma unroll 8
+      for (int r = q; r < RB; r += ng) sg += p[(size_t)r * st];
+    }
+    if (b) __syncthreads();
     gred[t] = sg;
     __syncthreads();
     if (q == 0 && d < D) {
       float tot = 0.0f;
-      for (int k = 0; k < ng; ++k) tot += gred[k * dp2 + d];
+      for (int k = 0; k < ng; ++k) tot += gred[k * min(dp, NT) + d0];
       const float zv = Z[(size_t)c * ldz + d];
       g[(size_t)c * ldg + d] = tot + (float)(zv * inv_s2);
-      pr = 0.5 * (double)zv * zv * inv_s2 + log_norm;
-    }
-  } else {
-    for (int d = t; d < D; d += 256) {
-      float sg = 0.0f;
-      for (int r = 0; r < RB; ++r) sg += wsg[((size_t)r * ldw + ci) * D + d];
-      const float zv = Z[(size_t)c * ldz + d];
-      g[(size_t)c * ldg + d] = sg + (float)(zv * inv_s2);
       pr += 0.5 * (double)zv * zv * inv_s2 + log_norm;
     }
   }
   CompSum u;  // this thread's row-split energy partials, compensated
-  for (int r = t; r < RB; r += 256) u.add(wsu[(size_t)r * ldw + ci]);
-  red[t] = pr;
-  us[t] = u.s;
-  uc[t] = u.c;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (t < o) {
-      red[t] += red[t + o];
-      CompSum a, b;
-      a.s = us[t];
-      a.c = uc[t];
-      b.s = us[t + o];
-      b.c = uc[t + o];
-      a.add(b);
-      us[t] = a.s;
-      uc[t] = a.c;
-    }
-    __syncthreads();
+  for (int r = t; r < RB; r += NT) u.add(wsu[(size_t)r * ldw + ci]);
+  pr = wave_sum(pr);
+#pragma unroll
+  for (int o = NAX_WAVE / 2; o > 0; o >>= 1) {
+    CompSum v;
+    v.s = __shfl_xor(u.s, o, NAX_WAVE);
+    v.c = __shfl_xor(u.c, o, NAX_WAVE);
+    u.add(v);
   }
+  if (lane == 0) {
+    us[wave] = u.s;
+    uc[wave] = u.c;
+    pw[wave] = pr;
+  }
+  __syncthreads();
   if (t == 0) {
     CompSum tot;
-    tot.s = us[0];
-    tot.c = uc[0];
-    tot.add(red[0]);
+    double prior = 0.0;
+    for (int w = 0; w < NW; ++w) {
+      CompSum v;
+      v.s = us[w];
+      v.c = uc[w];
+      tot.add(v);
+      prior += pw[w];
+    }
+    tot.add(prior);
     tot.add(u_offset);
     pe[c] = tot.value();
   }
@@ -367,7 +370,7 @@ struct LogisticPotential : Potential {
     if (e != hipSuccess) return e;
     const double inv_s2 = 1.0 / (prior_scale * prior_scale);
     const double log_norm = std::log(std::sqrt(2.0 * M_PI) * prior_scale);
-    hipLaunchKernelGGL(logit_reduce, dim3(C), dim3(256), 0, s, wsg, wsu, RB, C, d, z, ldz,
+    hipLaunchKernelGGL(logit_reduce, dim3(C), dim3(reduce_threads(C)), 0, s, wsg, wsu, RB, C, d, z, ldz,
                        inv_s2, log_norm, 0.0, pe, g, ldg, nullptr, nullptr, 0, 0);
     return hipGetLastError();
   }
@@ -650,7 +653,7 @@ extern "C" int nax_logistic_potential_grad_noalloc(const float* d_x, const float
   if (e == hipSuccess) {
     const double inv_s2 = 1.0 / (prior_scale * prior_scale);
     const double log_norm = std::log(std::sqrt(2.0 * M_PI) * prior_scale);
-    hipLaunchKernelGGL(logit_reduce, dim3(count), dim3(256), 0, s, wsg, wsu, RB, count, d, d_z,
+    hipLaunchKernelGGL(logit_reduce, dim3(count), dim3(reduce_threads(count)), 0, s, wsg, wsu, RB, count, d, d_z,
                        ld, inv_s2, log_norm, 0.0, d_pe, d_grad, ld, nullptr, nullptr, 0, 0);
     e = hipGetLastError();
   }

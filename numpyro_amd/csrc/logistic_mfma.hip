@@ -478,13 +478,6 @@ __global__ void abs_max_kernel(const float* __restrict__ X, int64_t n, unsigned*
   if ((threadIdx.x & 63) == 0) atomicMax(out, __float_as_uint(m));
 }
 
-// Fixed-order sum of the partials (+ Normal prior), defined in logistic.hip.
-__global__ void logit_reduce(const float* __restrict__ wsg, const double* __restrict__ wsu, int RB,
-                             int C, int D, const float* __restrict__ Z, int ldz, double inv_s2,
-                             double log_norm, double u_offset, double* __restrict__ pe,
-                             float* __restrict__ g, int ldg, const int* __restrict__ act,
-                             const int* __restrict__ nact, int nblk, int64_t ntile);
-
 struct LogisticMfma : Potential {
   int64_t n = 0, ntile = 0;
   int d = 0, dp = 0;
@@ -608,7 +601,7 @@ struct LogisticMfma : Potential {
     const double log_norm = std::log(std::sqrt(2.0 * M_PI) * prior_scale);
     // padded rows each added fp32(ln 2) to every chain's energy
     const double pad_u = (double)(ntile * 32 - n) * (double)0.693147180559945309f;
-    hipLaunchKernelGGL(logit_reduce, dim3(C), dim3(256), 0, s, wsg, wsu, RB, C, d, z, ldz,
+    hipLaunchKernelGGL(logit_reduce, dim3(C), dim3(reduce_threads(C)), 0, s, wsg, wsu, RB, C, d, z, ldz,
                        inv_s2, log_norm, -pad_u, pe, g, ldg, act, nact, nblk, ntile);
     return hipGetLastError();
   }

@@ -589,13 +589,6 @@ logit_split_kernel(const void* __restrict__ XA, const void* __restrict__ XB,
   if (h == 0 && cvalid) wsu[(size_t)rb * ldw + c0 + cl] = ut;
 }
 
-// Fixed-order sum of the partials (+ Normal prior), defined in logistic.hip.
-__global__ void logit_reduce(const float* __restrict__ wsg, const double* __restrict__ wsu, int RB,
-                             int C, int D, const float* __restrict__ Z, int ldz, double inv_s2,
-                             double log_norm, double u_offset, double* __restrict__ pe,
-                             float* __restrict__ g, int ldg, const int* __restrict__ act,
-                             const int* __restrict__ nact, int nblk, int64_t ntile);
-
 struct LogisticSplit : Potential {
   int64_t n = 0, ntile = 0;
   int d = 0, dp = 0;
@@ -754,7 +747,7 @@ struct LogisticSplit : Potential {
     // padded rows each added fp32(ln 2) to every chain's energy (split forms)
     const float pad = mode == kSplitFp8 ? log1pf(1.0f) : 0.693147180559945309f;
     const double pad_u = mode == kPlainF32 ? 0.0 : (double)(ntile * 32 - n) * (double)pad;
-    hipLaunchKernelGGL(logit_reduce, dim3(C), dim3(256), 0, s, wsg, wsu, RB, C, d, z, ldz, inv_s2,
+    hipLaunchKernelGGL(logit_reduce, dim3(C), dim3(reduce_threads(C)), 0, s, wsg, wsu, RB, C, d, z, ldz, inv_s2,
                        log_norm, -pad_u, pe, g, ldg, act, nact, nblk, ntile);
     return hipGetLastError();
   }

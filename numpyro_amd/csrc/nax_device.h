@@ -361,4 +361,14 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
+// Fixed-order sum of the logistic kernels' row-split partials and the prior,
+// one block per chain (logistic.hip).
+constexpr int kReduceThreads = 1024;
+inline int reduce_threads(int chains) { return chains > 512 ? 256 : kReduceThreads; }
+__global__ void logit_reduce(const float* __restrict__ wsg, const double* __restrict__ wsu, int RB,
+                             int C, int D, const float* __restrict__ Z, int ldz, double inv_s2,
+                             double log_norm, double u_offset, double* __restrict__ pe,
+                             float* __restrict__ g, int ldg, const int* __restrict__ act,
+                             const int* __restrict__ nact, int nblk, int64_t ntile);
+
 }  // namespace nax
