@@ -27,7 +27,8 @@
 // U and X^T R are added in r order at the end -- a heavy model's leaf then
 // takes ~1/R of the time, which is what the launch waits for.  The NUTS
 // state machine of a chain runs on its wave r = 0.  The autotuner picks
-// (KB, R).
+// (KB, R).  One evaluation outside a run, where no chain waits for another, has a
+// kernel of its own (hier_once_kernel).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -86,6 +87,35 @@ struct HierPipe {
   static constexpr int PF = (EPT >= 32) ? 1 : 2;
 };
 
+// U and dU of a chain at z from its likelihood part U_lik and, lane = column,
+// the column's X^T r (0 past D), on one wave.
+__device__ inline double hier_finish(const HierData& hd, int D, int lane, const float* z, float acc,
+                                     double U_lik, float* g) {
+  const float mu = z[D];
+  const PosTf tt = positive_tf((double)z[D + 1], hd.softplus != 0);
+  const float tau = hd.softplus ? (float)tt.x : expf(z[D + 1]);
+  const float eta = lane < D ? z[lane] : 0.0f;
+  // dU/deta = eta + tau acc, dU/dmu = mu + sum acc,
+  // dU/dlog tau = tau eta.acc + 2 tau^2 / (1 + tau^2) - 1
+  const double sum_acc = wave_sum((double)acc);
+  const double eta_acc = wave_sum((double)eta * acc);
+  const double eta2 = wave_sum((double)eta * eta);
+  if (lane < D) g[lane] = eta + tau * acc;
+  const double t2 = (double)tau * tau;
+  if (lane == 0) {
+    g[D] = (float)((double)mu + sum_acc);
+    // softplus: dtau/du (eta.acc + 2 tau / (1 + tau^2)) - d log|J| / du
+    g[D + 1] = hd.softplus
+        ? (float)(tt.dx * (eta_acc + 2.0 * (double)tau / (1.0 + t2)) - tt.dladj)
+        : (float)((double)tau * eta_acc + 2.0 * t2 / (1.0 + t2) - 1.0);
+  }
+  const double U = U_lik + 0.5 * eta2 + D * kLog2PiHalf          // eta ~ N(0,1)
+                   + 0.5 * (double)mu * mu + kLog2PiHalf          // mu ~ N(0,1)
+                   - (kLog2 - kLogPi_ - log1p(t2))                // HalfCauchy(1)
+                   - (hd.softplus ? tt.ladj : (double)z[D + 1]);  // log|J|
+  return U;
+}
+
 // Block-cooperative U and dU for the K chains of model i at z[c] (c = chain
 // index of the block's chain slot w: c = i K_model + sub K + w), each chain
 // on R waves (wave index w R + r).  Wave r = 0 of slot w ends with its own
@@ -118,11 +148,10 @@ __device__ double hier_group_eval(const HierData& hd, int i, int sub, const floa
   const int c = i * hd.K + sub * K + w;
   const float* z = zreq + (size_t)c * ldz;
   float* g = gout + (size_t)c * ldg;
-  const float mu = z[D];
-  const PosTf tt = positive_tf((double)z[D + 1], hd.softplus != 0);
-  const float tau = hd.softplus ? (float)tt.x : expf(z[D + 1]);
-  const float eta = lane < D ? z[lane] : 0.0f;
-  if (r == 0) sh.beta[w][lane] = lane < D ? mu + tau * eta : 0.0f;
+  if (r == 0) {
+    const float tau = hd.softplus ? (float)positive_tf((double)z[D + 1], true).x : expf(z[D + 1]);
+    sh.beta[w][lane] = lane < D ? z[D] + tau * z[lane] : 0.0f;
+  }
   // columns [D, D4) of both buffers stay zero for the whole evaluation
   for (int e = threadIdx.x; e < 2 * TR * 4; e += NT) {
     const int b = e / (TR * 4), rr = (e / 4) % TR, cc = D + (e & 3);
@@ -232,25 +261,7 @@ __device__ double hier_group_eval(const HierData& hd, int i, int sub, const floa
   } else {
     U_lik = wave_sum(ul);
   }
-  // chain w's own gradient: dU/deta = eta + tau acc, dU/dmu = mu + sum acc,
-  // dU/dlog tau = tau eta.acc + 2 tau^2 / (1 + tau^2) - 1
-  const double sum_acc = wave_sum((double)acc);
-  const double eta_acc = wave_sum((double)eta * acc);
-  const double eta2 = wave_sum((double)eta * eta);
-  if (lane < D) g[lane] = eta + tau * acc;
-  const double t2 = (double)tau * tau;
-  if (lane == 0) {
-    g[D] = (float)((double)mu + sum_acc);
-    // softplus: dtau/du (eta.acc + 2 tau / (1 + tau^2)) - d log|J| / du
-    g[D + 1] = hd.softplus
-        ? (float)(tt.dx * (eta_acc + 2.0 * (double)tau / (1.0 + t2)) - tt.dladj)
-        : (float)((double)tau * eta_acc + 2.0 * t2 / (1.0 + t2) - 1.0);
-  }
-  const double U = U_lik + 0.5 * eta2 + D * kLog2PiHalf          // eta ~ N(0,1)
-                   + 0.5 * (double)mu * mu + kLog2PiHalf          // mu ~ N(0,1)
-                   - (kLog2 - kLogPi_ - log1p(t2))                // HalfCauchy(1)
-                   - (hd.softplus ? tt.ladj : (double)z[D + 1]);  // log|J|
-  return U;
+  return hier_finish(hd, D, lane, z, acc, U_lik, g);
 }
 
 template <int K, int R>
@@ -264,6 +275,292 @@ hier_eval_kernel(HierData hd, const float* __restrict__ zreq, int ldz, double* _
   const double u = hier_group_eval<K, R>(hd, i, sub, zreq, ldz, gout, ldg, sh);
   const int wa = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0 && wa % R == 0) pe[i * hd.K + sub * K + wa / R] = u;
+}
+
+// fourth word of a buffer descriptor: plain 32-bit data
+constexpr int kBufferWord3 = 0x00027000;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// One-shot evaluation: waves of a block and rows of a wave's tile (1024 models x
+// 4 chains, models whole: 8 x 32 116 us a pass, 4 x 64 130 us; in an earlier
+// form 16 x 16 166, 8 x 16 152, 8 x 32 136, 4 x 64 160, 4 x 32 167, 2 x 64 218).
+constexpr int kOnceWaves = 8, kOnceRows = 32;
+static_assert(kOnceRows % 32 == 0 && kOnceRows <= 64, "tile layout");
+// A model above 1 / 256 of all elements (one CU's part) is split into items: 1024
+// models of up to 5000 x 64 are then whole, where items of half and of an eighth of
+// that cost 6 and 15 us of starting blocks and combining (116 us a pass), and 60
+// models x 4 chains still fill the chip (345 -> 112 us a pass).  No item is split
+// below 64 KB, two rounds of a block's tiles.
+constexpr double kOnceItems = 256.0, kOnceItemMin = 16384.0;
+
+// Rows [row0, row0 + rows) of a model; slot: where the partial sums go, -1 when
+// the item is its whole model.
+struct HierItem {
+  int64_t row0, rows;
+  int model, slot;
+};
+// A model of several items and its first slot.
+struct HierSplit {
+  int model, slot, count;
+};
+
+// U and dU of the K chains of one item's rows, once: the rows in tiles of TR over
+// W waves, each wave evaluating all K chains on its tiles, so X_i is read
+// once and a tile's bytes leave LDS once for each product instead of once per
+// chain.  The tiles are the wave's own (no barrier in the loop): loaded into
+// registers one tile ahead, stored into LDS, then
+//   logits     lane = row: one v_mfma_f32_4x4x1 (16 blocks of 4 rows x 4 chains)
+//              per column and 4 chains: the same four interleaved sums of fused
+//              multiply-adds as hier_group_eval, bit for bit
+//   residuals  lane = (4 rows, chain) of those accumulators
+//   X^T R      lane = column: one v_mfma_f32_4x4x1 per row and 4 chains
+// and the waves' partial sums are added in wave order.  Bound: the reads of X and,
+// in a block, the start of its first tiles and the finish of its chains (1024
+// models x 4 chains, 350 MB: 220 us with a wave per chain on a shared tile, every
+// chain reading the tile from LDS and one tile of dword loads in flight; 98 us
+// now, against 75 us for a copy of as many bytes).
+template <int K, int W, int TR>
+__global__ void __launch_bounds__(64 * W, 2)
+hier_once_kernel(HierData hd, const HierItem* __restrict__ items, const float* __restrict__ zreq,
+                 int ldz, double* __restrict__ pe, float* __restrict__ gout, int ldg,
+                 float* __restrict__ part_g, double* __restrict__ part_u) {
+  constexpr int SETS = (K + 3) / 4;     // groups of 4 chains
+  constexpr int SG = SETS < 2 ? 1 : 2;  // sets at a time: 16 SG accumulator registers
+  constexpr int NC = 4 * SETS;
+  constexpr int NLD = TR * kHierMaxD / 256;
+  // each wave's X tile, at the end its partial X^T R ([chain][column])
+  __shared__ __attribute__((aligned(16))) float xs_all[W][TR * kHierLd];
+  __shared__ __attribute__((aligned(16))) float beta[NC][kHierLd];  // unused chains: 0
+  __shared__ __attribute__((aligned(16))) float res[W][NC][TR + 4];   // sigmoid(l) - y
+  __shared__ __attribute__((aligned(16))) float ys[W][TR];
+  __shared__ double rul[W][NC];                                       // partial U
+  const HierItem it = items[blockIdx.x];
+  const int i = it.model;
+  const int wa = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int D = hd.dims[i];
+  const int64_t N = it.rows;
+  const int ntiles = (int)((N + TR - 1) / TR);
+  const float* X = hd.x + hd.elt_off[i] + it.row0 * D;
+  const float* Y = hd.y + hd.row_off[i] + it.row0;
+  for (int q = wa; q < NC; q += W) {
+    float b = 0.0f;
+    if (q < K && lane < D) {
+      const float* z = zreq + (size_t)(i * K + q) * ldz;
+      const float tau = hd.softplus ? (float)positive_tf((double)z[D + 1], true).x : expf(z[D + 1]);
+      b = z[D] + tau * z[lane];
+    }
+    beta[q][lane] = b;
+  }
+  // The wave's own tile.  Its TR D elements are contiguous in memory: loaded and
+  // stored to LDS 16 bytes a lane, chunk lane + 64 j of the tile.  Rows are SD
+  // apart in LDS: D a multiple of 8 takes 4 floats of padding, which spreads the
+  // rows over the banks; any other D is conflict-free (or 2-way) as it is.
+  float* xs = xs_all[wa];
+  const bool quad = (D & 3) == 0;
+  const int SD = (D & 7) == 0 ? D + 4 : D;
+  const int nld = (TR * D + 255) / 256;  // 16-byte loads of a tile
+  int dst[NLD];
+#pragma unroll
+  for (int j = 0; j < NLD; ++j) {
+    const int e = 4 * (lane + 64 * j);
+    dst[j] = SD == D ? e : e + 4 * (e / D);
+  }
+  f32x4 px[NLD];
+  float py = 0.0f;
+  const int full = (int)(N / TR);  // tiles of TR rows; at most one more, of fewer
+  // Every load of a full tile is issued, without a branch: what lies past the
+  // tile's TR D elements (16 bytes never straddle that end) or past the last full
+  // tile reads as 0 and takes no memory access.
+  auto load = [&](int t) {
+    const int64_t r0 = (int64_t)t * TR;
+    const int ok = t < full ? 4 * TR : 0;
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(X + r0 * D), 0, ok * D,
+                                                      kBufferWord3);
+    const auto ry =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Y + r0), 0, ok, kBufferWord3);
+#pragma unroll
+    for (int j = 0; j < NLD; ++j)
+      px[j] = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, 16 * (lane + 64 * j), 0, 0));
+    py = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ry, 4 * lane, 0, 0));
+  };
+  load(wa);
+  const int j4 = lane & 3, b4 = lane >> 2;  // chain of a set, block of 4 rows / columns
+  constexpr int RV = TR / 16;  // rows a lane takes the residuals of
+  const bool upper = lane >= TR;
+  const int rl = 4 * b4 % TR + (upper ? RV : 0);
+  f32x4 acc[SETS];    // dU/dbeta of columns 4 b4 .. 4 b4 + 3, chain 4 s + j4
+  double ul[SETS];    // likelihood part of U, chain 4 s + j4
+#pragma unroll
+  for (int s = 0; s < SETS; ++s) {
+    acc[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    ul[s] = 0.0;
+  }
+  __syncthreads();  // beta
+  for (int t = wa; t < ntiles; t += W) {
+    const int rows = (int)min<int64_t>(TR, N - (int64_t)t * TR);
+    if (t < full) {
+#pragma unroll
+      for (int j = 0; j < NLD; ++j)
+        if (j < nld) *reinterpret_cast<f32x4*>(xs + dst[j]) = px[j];
+      if (lane < TR) ys[wa][lane] = py;
+      load(t + W);  // in flight during the compute below
+    } else {  // the last rows, one number a lane; zeros after them
+      const int64_t r0 = (int64_t)t * TR;
+      const int ne = rows * D;
+      for (int e = lane; e < TR * D; e += 64)
+        xs[SD == D ? e : e + 4 * (e / D)] = e < ne ? X[r0 * D + e] : 0.0f;
+      if (lane < TR) ys[wa][lane] = lane < rows ? Y[r0 + lane] : 0.0f;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float yv[RV];
+#pragma unroll
+    for (int v = 0; v < RV; ++v) yv[v] = ys[wa][rl + v];
+    // logits: lane = row (at TR = 32 twice), four interleaved sums
+    const float* xr = xs + lane % TR * SD;
+#pragma unroll
+    for (int s0 = 0; s0 < SETS; s0 += SG) {
+      f32x4 l[SG][4];
+#pragma unroll
+      for (int s = 0; s < SG; ++s)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) l[s][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (quad) {
+#pragma unroll 2
+        for (int q = 0; q < D; q += 4) {
+          const f32x4 xv = *reinterpret_cast<const f32x4*>(xr + q);
+#pragma unroll
+          for (int s = 0; s < SG; ++s) {
+            const f32x4 bv = *reinterpret_cast<const f32x4*>(&beta[4 * (s0 + s) + j4][q]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              l[s][k] = __builtin_amdgcn_mfma_f32_4x4x1f32(xv[k], bv[k], l[s][k], 0, 0, 0);
+          }
+        }
+      } else {
+#pragma unroll 2
+        for (int q = 0; q < D - 3; q += 4) {
+#pragma unroll
+          for (int s = 0; s < SG; ++s) {
+            const f32x4 bv = *reinterpret_cast<const f32x4*>(&beta[4 * (s0 + s) + j4][q]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              l[s][k] = __builtin_amdgcn_mfma_f32_4x4x1f32(xr[q + k], bv[k], l[s][k], 0, 0, 0);
+          }
+        }
+        const int q = D & ~3;
+#pragma unroll
+        for (int s = 0; s < SG; ++s) {
+          const f32x4 bv = *reinterpret_cast<const f32x4*>(&beta[4 * (s0 + s) + j4][q]);
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+            l[s][k] = __builtin_amdgcn_mfma_f32_4x4x1f32(q + k < D ? xr[q + k] : 0.0f, bv[k],
+                                                         l[s][k], 0, 0, 0);
+        }
+      }
+      // residuals, RV rows a lane from row rl; rows past `rows` get 0
+#pragma unroll
+      for (int s = 0; s < SG; ++s)
+#pragma unroll
+        for (int v = 0; v < RV; ++v) {
+          f32x4 lv;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            lv[k] = l[s][k][v];
+            if (RV < 4 && upper) lv[k] = l[s][k][(v + RV) % 4];
+          }
+          float r, u;
+          logistic_terms_f((lv[0] + lv[1]) + (lv[2] + lv[3]), yv[v], r, u);
+          const bool ok = rl + v < rows;
+          res[wa][4 * (s0 + s) + j4][rl + v] = ok ? r : 0.0f;
+          ul[s0 + s] += ok ? (double)u : 0.0;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // X^T R: lane = column, four interleaved sums over the tile's rows
+    const float* xc = xs + lane;  // lanes past D: any number, not used
+#pragma unroll
+    for (int s0 = 0; s0 < SETS; s0 += SG) {
+      f32x4 p[SG][4];
+#pragma unroll
+      for (int s = 0; s < SG; ++s)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[s][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+      for (int n4 = 0; n4 < TR / 4; ++n4) {
+#pragma unroll
+        for (int s = 0; s < SG; ++s) {
+          const f32x4 rv =
+              *reinterpret_cast<const f32x4*>(&res[wa][4 * (s0 + s) + j4][4 * n4]);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            p[s][k] = __builtin_amdgcn_mfma_f32_4x4x1f32(xc[(4 * n4 + k) * SD], rv[k],
+                                                         p[s][k], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < SG; ++s)
+        acc[s0 + s] += (p[s][0] + p[s][1]) + (p[s][2] + p[s][3]);
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < SETS; ++s) {
+    *reinterpret_cast<f32x4*>(xs + (4 * s + j4) * kHierMaxD + 4 * b4) = acc[s];
+#pragma unroll
+    for (int o = 4; o < 64; o <<= 1) ul[s] += __shfl_xor(ul[s], o, 64);
+    if (b4 == 0) rul[wa][4 * s + j4] = ul[s];
+  }
+  __syncthreads();
+  for (int q = wa; q < K; q += W) {
+    const int c = i * K + q;
+    const float* z = zreq + (size_t)c * ldz;
+    float* g = gout + (size_t)c * ldg;
+    float a = 0.0f;
+    double u = 0.0;
+#pragma unroll
+    for (int v = 0; v < W; ++v) {
+      a += xs_all[v][q * kHierMaxD + lane];
+      u += rul[v][q];
+    }
+    if (it.slot >= 0) {
+      const size_t p = (size_t)it.slot * K + q;
+      part_g[p * kHierMaxD + lane] = a;
+      if (lane == 0) part_u[p] = u;
+    } else {
+      u = hier_finish(hd, D, lane, z, lane < D ? a : 0.0f, u, g);
+      if (lane == 0) pe[c] = u;
+    }
+  }
+}
+
+// U and dU of the split models from their items' partial sums, added in row
+// order: a wave per chain.
+__global__ void __launch_bounds__(64)
+hier_combine_kernel(HierData hd, const HierSplit* __restrict__ splits,
+                    const float* __restrict__ part_g, const double* __restrict__ part_u,
+                    const float* __restrict__ zreq, int ldz, double* __restrict__ pe,
+                    float* __restrict__ gout, int ldg) {
+  const HierSplit sp = splits[blockIdx.x / hd.K];
+  const int q = blockIdx.x % hd.K, lane = threadIdx.x;
+  const int D = hd.dims[sp.model];
+  float a = 0.0f;
+  double u = 0.0;
+#pragma unroll 8
+  for (int t = 0; t < sp.count; ++t) {
+    const size_t p = (size_t)(sp.slot + t) * hd.K + q;
+    a += part_g[p * kHierMaxD + lane];
+    u += part_u[p];
+  }
+  const int c = sp.model * hd.K + q;
+  u = hier_finish(hd, D, lane, zreq + (size_t)c * ldz, lane < D ? a : 0.0f, u,
+                  gout + (size_t)c * ldg);
+  if (lane == 0) pe[c] = u;
 }
 
 // One block per (model, chain subset): K chain slots of R waves each.  Wave
@@ -334,8 +631,16 @@ struct HierPotential : Potential {
   int64_t* row_off = nullptr;
   int64_t* elt_off = nullptr;
   double flops = 0.0, bytes = 0.0;
+  // unforced evaluation: items heaviest first, the models of several items, and
+  // the partial sums of those items
+  HierItem* items = nullptr;
+  HierSplit* splits = nullptr;
+  float* part_g = nullptr;
+  double* part_u = nullptr;
+  int n_items = 0, n_splits = 0;
 
   ~HierPotential() override {
+    hipFree(items); hipFree(splits); hipFree(part_g); hipFree(part_u);
     hipFree(order); hipFree(dims); hipFree(cdims); hipFree(row_off); hipFree(elt_off);
   }
   int dim() const override { return maxd + 2; }
@@ -391,14 +696,26 @@ struct HierPotential : Potential {
   hipError_t eval(hipStream_t s, const float* z, int ldz, int Cn, double* pe, float* g,
                   int ldg) override {
     if (Cn != C || ldz < maxd + 2 || ldg < maxd + 2) return hipErrorInvalidValue;
-    // one evaluation of every chain: one wave per chain unless a shape was
-    // fixed (C4 at fixed positions: 0.224 ms with one wave per chain, 0.299
-    // with two, 0.255 with four -- the waves per chain pay off only on the
-    // heavy models' chains that the persistent launch waits for)
-    const int w = waves(), r = forced ? rw : 1;
-    const dim3 grid(groups * (hd.K / w));
+    // one evaluation of every chain, unless a shape was fixed: then that shape's
+    // evaluation, whose sums are in the order of the persistent launch's
     bool launched = false;
     mark_begin(s);
+    if (!forced) {
+#define NAX_K(KV)                                                                             \
+  if (hd.K == KV)                                                                             \
+    hipLaunchKernelGGL((hier_once_kernel<KV, kOnceWaves, kOnceRows>), dim3(n_items),          \
+                       dim3(64 * kOnceWaves), 0, s, hd, items, z, ldz, pe, g, ldg, part_g,    \
+                       part_u);
+      NAX_K(1) NAX_K(2) NAX_K(4) NAX_K(8) NAX_K(16)
+#undef NAX_K
+      if (n_splits)
+        hipLaunchKernelGGL(hier_combine_kernel, dim3(n_splits * hd.K), dim3(64), 0, s, hd, splits,
+                           part_g, part_u, z, ldz, pe, g, ldg);
+      mark_end(s);
+      return hipGetLastError();
+    }
+    const int w = waves(), r = rw;
+    const dim3 grid(groups * (hd.K / w));
 #define NAX_KR(KV, RV)                                                                        \
   if (!launched && w == KV && r == RV) {                                                      \
     hipLaunchKernelGGL((hier_eval_kernel<KV, RV>), grid, dim3(64 * KV * RV), 0, s, hd, z,     \
@@ -532,7 +849,35 @@ Potential* make_hier(const float* x, const float* y, const int64_t* d_row_off,
   std::vector<int> ord(groups);
   std::iota(ord.begin(), ord.end(), 0);
   std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return w[a] > w[b]; });
+  std::vector<HierItem> items;
+  std::vector<HierSplit> splits;
+  const double share = std::max(work / kOnceItems, kOnceItemMin);
+  int slots = 0;
+  for (int i : ord) {
+    const int64_t n = hrow[i + 1] - hrow[i];
+    const int64_t tiles = (n + kOnceRows - 1) / kOnceRows;
+    const int64_t parts = std::min<int64_t>(tiles, (int64_t)std::ceil(w[i] / share));
+    if (parts > 1) splits.push_back({i, slots, (int)parts});
+    for (int64_t t = 0; t < parts; ++t) {
+      const int64_t a = tiles * t / parts * kOnceRows;
+      const int64_t b = std::min<int64_t>(n, tiles * (t + 1) / parts * kOnceRows);
+      items.push_back({a, b - a, i, parts > 1 ? slots++ : -1});
+    }
+  }
+  std::stable_sort(items.begin(), items.end(), [&](const HierItem& a, const HierItem& b) {
+    return a.rows * hd_dims[a.model] > b.rows * hd_dims[b.model];
+  });
+  p->n_items = (int)items.size();
+  p->n_splits = (int)splits.size();
   hipError_t e = hipMalloc(&p->order, sizeof(int) * groups);
+  if (e == hipSuccess) e = hipMalloc(&p->items, sizeof(HierItem) * items.size());
+  if (e == hipSuccess && slots) {
+    e = hipMalloc(&p->splits, sizeof(HierSplit) * splits.size());
+    if (e == hipSuccess) e = hipMalloc(&p->part_g, sizeof(float) * slots * K * kHierMaxD);
+    if (e == hipSuccess) e = hipMalloc(&p->part_u, sizeof(double) * slots * K);
+    if (e == hipSuccess) e = hipMemcpy(p->splits, splits.data(), sizeof(HierSplit) * splits.size(), hipMemcpyHostToDevice);
+  }
+  if (e == hipSuccess) e = hipMemcpy(p->items, items.data(), sizeof(HierItem) * items.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMalloc(&p->dims, sizeof(int) * groups);
   if (e == hipSuccess) e = hipMalloc(&p->cdims, sizeof(int) * C);
   if (e == hipSuccess) e = hipMalloc(&p->row_off, sizeof(int64_t) * (groups + 1));
