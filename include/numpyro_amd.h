@@ -173,8 +173,10 @@ int nax_model_hier(nax_sampler* h, const float* d_x, const float* d_y, const int
 
 /* nax_model_logistic with the kernel choice for fp32 storage: 0 = auto
  * (one wavefront per chain in a persistent launch for <= 16 chains on
- * n*d <= 2^20, d <= 64; otherwise the VALU tile kernel or, from 32 chains
- * up, the matrix-core kernel, whichever the autotuner times faster), 1 = VALU
+ * n*d <= 2^20, d <= 64; otherwise, for d <= 256, row tiles on the fp32 matrix
+ * cores below 32 chains, the VALU tile kernel or the matrix-core kernel,
+ * whichever the autotuner times faster, up to 128 and the matrix-core kernel
+ * above; the VALU tile kernel for 257 <= d <= 320), 1 = VALU
  * tile kernel, 2 = matrix cores (X Z^T in fp32; X^T R by two fp16 terms per
  * factor where rows and column ranges allow, else fp32), 3 = one wavefront per
  * chain.  bf16 storage

@@ -14,7 +14,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 OUT = os.path.join(HERE, "libnumpyro_amd.so")
 SOURCES = ["sampler.hip", "logistic.hip", "logistic_mfma.hip", "logistic_split.hip",
-           "logistic_chain.hip", "sv.hip", "hier.hip", "diagnostics.hip", "ecs.hip"]
+           "logistic_rows.hip", "logistic_chain.hip", "sv.hip", "hier.hip", "diagnostics.hip", "ecs.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

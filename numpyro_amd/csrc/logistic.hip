@@ -26,8 +26,6 @@
 
 namespace nax {
 
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + __expf(-x)); }
-
 // ---- X storage forms of the tile kernel ----------------------------------------
 // fp32: X as given.  FP8: X[n][d] = e4m3(code[n][d]) * scale[d], the OCP
 // e4m3fn byte (1 sign, 4 exponent bits with bias 7, 3 mantissa bits; no
@@ -467,12 +465,15 @@ Potential* make_logistic_mfma(const float* x, const float* y, int64_t n, int d,
                               double prior_scale, bool single, hipStream_t s,
                               std::string* err);
 
+Potential* make_logistic_rows(const float* x, const float* y, int64_t n, int d,
+                              double prior_scale);
+
 int64_t logistic_split_min_rows();
 Potential* make_logistic_split(const float* x, const uint8_t* codes, const float* scales,
                                const float* y, int64_t n, int d, double prior_scale,
                                int num_chains, hipStream_t s, std::string* err);
 
-// fuse_variant: 0 = auto (fp32: matrix cores when num_chains >= 32), 1 = VALU tile
+// fuse_variant: 0 = auto (fp32: row tiles below 32 chains, else matrix cores), 1 = VALU tile
 // kernel, 2 = matrix cores, 3 = a group of wavefronts per chain.  bf16 always runs on
 // the matrix cores: 0 or 4 keep one X copy (bf16 residuals in X^T R), 2 keeps
 // a second, fp16 copy for X^T R with fp16 residuals.
@@ -520,6 +521,13 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
     *err = "the fp32 logistic tile kernel supports dim <= 320";
     return nullptr;
   }
+  // up to 31 chains: wave-owned row tiles on the fp32 matrix cores (a pass, against
+  // the tile kernel at its best row split: 581,012 x 55, 1, 8, 16, 31 chains 66, 79,
+  // 115, 187 us against 105, 118, 185, 325; 1,000,000 x 256, 1, 16, 31 chains 0.29,
+  // 0.77, 1.49 ms against 1.02, 1.94, 3.83; 2,000 x 100, 4 chains both at the host's
+  // 70).  Its LDS tiles hold 256 columns.
+  if (!fp8 && fuse_variant == 0 && num_chains >= 1 && num_chains < 32 && d <= 256)
+    return make_logistic_rows(x, y, n, d, prior_scale);
   auto* p = new LogisticPotential();
   p->x = x;
   p->y = y;
@@ -542,8 +550,9 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
     }
   }
   if (fuse_variant != 0 || num_chains < 1) return p;
-  // Autotuner ("auto" kernel): row splits of the tile kernel, and for 32 <=
-  // C <= 128 the tile kernel against the matrix-core kernel, each timed over a
+  // Autotuner ("auto" kernel): row splits of the tile kernel (fp8 of few rows, fp32
+  // of 257 to 320 columns or 32 to 128 chains), and for 32 <= C <= 128 the tile
+  // kernel against the matrix-core kernel, each timed over a
   // few evaluations of all C chains at z = 0; the fastest is kept.
   const int C = num_chains;
   const int ld = (d + 63) / 64 * 64;

@@ -297,6 +297,8 @@ __device__ __forceinline__ void logit_terms(float l, float y, float& r, float& u
   u = fmaf(__builtin_amdgcn_logf(d), 0.693147180559945309f, fmaf(-y, l, pos ? l : 0.0f));
 }
 
+__device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + __expf(-x)); }
+
 // max(x, 0) + log1p(exp(-|x|))  (distributions/util.py:317-320)
 __device__ __forceinline__ float softplusf_(float x) {
   return fmaxf(x, 0.0f) + log1pf(__expf(-fabsf(x)));
