@@ -59,6 +59,7 @@ struct EcsArgs {
   double LL;
 };
 
+template <int NW>
 __device__ __forceinline__ double block_sum(double v, double* red) {
   v = wave_sum(v);
   const int wv = threadIdx.x / NAX_WAVE, ln = threadIdx.x % NAX_WAVE;
@@ -66,7 +67,7 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   if (ln == 0) red[wv] = v;
   __syncthreads();
   double t = 0;
-  for (int i = 0; i < kEcsThreads / NAX_WAVE; ++i) t += red[i];
+  for (int i = 0; i < NW; ++i) t += red[i];
   return t;
 }
 
@@ -178,6 +179,102 @@ __global__ void ecs_reduce_kernel(const double* part, int nsplit, int64_t len, d
 
 // ---- the subsampled potential ------------------------------------------------
 
+// hd[c] = H delta_c, delta_c = z_c - bref, for kProxyChains chains per workgroup
+// (slots of act when a list is given), so that a read of H (d^2 doubles, from
+// L2) serves all of them; a workgroup per chain read it once per chain, inside
+// the evaluation and after all of its gathers.  Threads: 256 columns of H
+// (symmetric, so column reads are coalesced) times 4 quarters of its rows, 16
+// loads in flight each.  1024 chains, d = 256: 7 us.
+constexpr int kProxyChains = 4, kProxyParts = 4;
+__global__ __launch_bounds__(kEcsThreads * kProxyParts) void ecs_proxy_kernel(
+    EcsArgs a, const float* __restrict__ z, int ldz, int C, const int* act, const int* nact,
+    double* __restrict__ hd) {
+  __shared__ double dlt[kEcsMaxD][kProxyChains];
+  __shared__ double part[kProxyParts][kProxyChains][kEcsThreads];
+  const int d = a.d, tid = threadIdx.x % kEcsThreads, pt = threadIdx.x / kEcsThreads;
+  const int n = act ? min(*nact, C) : C;
+  const int s0 = blockIdx.x * kProxyChains;
+  if (s0 >= n) return;
+  int ch[kProxyChains];
+#pragma unroll
+  for (int u = 0; u < kProxyChains; ++u) {
+    const int s = min(s0 + u, n - 1);
+    ch[u] = act ? act[s] : s;
+  }
+  for (int k = threadIdx.x; k < d; k += kEcsThreads * kProxyParts)
+#pragma unroll
+    for (int u = 0; u < kProxyChains; ++u)
+      dlt[k][u] = (double)z[(int64_t)ch[u] * ldz + k] - a.bref[k];
+  __syncthreads();
+  const int l0 = (int)((int64_t)d * pt / kProxyParts), l1 = (int)((int64_t)d * (pt + 1) / kProxyParts);
+  for (int k0 = 0; k0 < d; k0 += kEcsThreads) {
+    const int k = min(k0 + tid, d - 1);
+    double acc[kProxyChains] = {};
+    int l = l0;
+    for (; l + 16 <= l1; l += 16) {
+      double h[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) h[i] = a.H[(int64_t)(l + i) * d + k];
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+#pragma unroll
+        for (int u = 0; u < kProxyChains; ++u) acc[u] += h[i] * dlt[l + i][u];
+    }
+    for (; l < l1; ++l) {
+      const double h = a.H[(int64_t)l * d + k];
+#pragma unroll
+      for (int u = 0; u < kProxyChains; ++u) acc[u] += h * dlt[l][u];
+    }
+#pragma unroll
+    for (int u = 0; u < kProxyChains; ++u) part[pt][u][tid] = acc[u];
+    __syncthreads();
+    // quarter pt adds chain pt's four parts
+    static_assert(kProxyParts == kProxyChains, "one chain per quarter");
+    if (s0 + pt < n && k0 + tid < d) {
+      double t = 0.0;
+#pragma unroll
+      for (int i = 0; i < kProxyParts; ++i) t += part[i][pt][tid];
+      hd[(int64_t)ch[pt] * d + k0 + tid] = t;
+    }
+    __syncthreads();
+  }
+}
+
+// Lane l reads lane l ^ 4 (the other quad of its eight lanes) / l ^ 8.
+__device__ __forceinline__ float lane_xor4(float v) {
+  const int x = __float_as_int(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, x, 0x104, 0xF, 0x5, false);  // row_shl:4
+  return __int_as_float(__builtin_amdgcn_update_dpp(lo, x, 0x114, 0xF, 0xA, false));  // row_shr:4
+}
+__device__ __forceinline__ float lane_xor8(float v) { return dpp_mov<0x128>(v); }  // row_ror:8
+
+// Sums over the wave of ROWS values per lane; lane l receives the sum of value
+// l % ROWS.  While values are left each step pairs lanes, one keeping the even
+// values and the other the odd ones, so that ROWS = 16 takes 15 exchanges
+// instead of 16 times 4.  The additions are those of wave_sum, in its order.
+template <int ROWS>
+__device__ __forceinline__ float rows_sum(float (&s)[ROWS], int ln) {
+  static_assert(ROWS == 8 || ROWS == 16, "rows of a wave's step");
+#pragma unroll
+  for (int b = 0, n = ROWS; n > 1; ++b, n /= 2) {
+    const bool odd = (ln >> b) & 1;
+#pragma unroll
+    for (int j = 0; j < n / 2; ++j) {
+      const float keep = odd ? s[2 * j + 1] : s[2 * j];
+      const float give = odd ? s[2 * j] : s[2 * j + 1];
+      const float got = b == 0   ? dpp_mov<dpp::kXor1>(give)
+                        : b == 1 ? dpp_mov<dpp::kXor2>(give)
+                        : b == 2 ? lane_xor4(give)
+                                 : lane_xor8(give);
+      s[j] = keep + got;
+    }
+  }
+  float t = s[0];
+  if constexpr (ROWS == 8) t += lane_xor8(t);
+  t += __shfl_xor(t, 16, NAX_WAVE);
+  return t + __shfl_xor(t, 32, NAX_WAVE);
+}
+
 // One workgroup per chain (act[blockIdx.x] when a list is given), one pass
 // over the subsample.  Each wavefront takes ROWS rows at a time, lanes
 // over the coordinates (the row values stay in registers), reduces l = x.beta
@@ -186,16 +283,23 @@ __global__ void ecs_reduce_kernel(const double* part, int nsplit, int64_t len, d
 // n/m (1 - n/m (diff_j - mean)), is n/m (1 + n/m mean) - (n/m)^2 diff_j, so
 // the gradient needs only S1 = sum c_j x_j and S2 = sum diff_j c_j x_j, both
 // accumulated from the registers while the mean is still unknown.
-// NCH: 64-column chunks of a row held in registers (d <= 64 NCH); ROWS rows
-// per wavefront step (fewer for wide rows, to stay within 128 VGPRs).
-template <int NCH, int ROWS>
-__global__ __launch_bounds__(kEcsThreads, NCH <= 4 ? 4 : 2) void ecs_eval_kernel(
+// NCH: 64-column chunks of a row held in registers (64 (NCH - 1) < d <= 64 NCH
+// up to NCH = 4).
+//
+// Bound: the gathered rows.  The fp64 terms (an exp, a log1p, a division) cost a
+// wave the same for 4 rows as for 64, and with 4 rows a step they and the
+// reductions of single rows took as long as the gathers; 16 rows a step share
+// them, at two waves per SIMD, with the next step's rows and records and the
+// indices of the one after in flight.  1024 chains of m = 1000, 2,000,000 x 256
+// (1.05 GB gathered, 5.4 TB/s): 299 us with H delta inside -> 193;
+// 512 chains x 128 columns, m = 1000: 58 us, 16 chains x 130: 30 us.
+template <int NCH, int ROWS, int NW>
+__global__ __launch_bounds__(NAX_WAVE * NW, NCH == 1 ? 3 : 2) void ecs_eval_kernel(
     EcsArgs a, const int* __restrict__ idx_all, const float* __restrict__ z, int ldz,
-    const int* act, const int* nact, double* pe, float* g, int ldg) {
-  constexpr int NW = kEcsThreads / NAX_WAVE;
-  __shared__ float beta[kEcsMaxD];
-  __shared__ double dlt[kEcsMaxD];
-  __shared__ double part[2][NW][kEcsMaxD];
+    const double* __restrict__ hd, const int* act, const int* nact, double* pe, float* g,
+    int ldg) {
+  constexpr int NT = NAX_WAVE * NW;
+  __shared__ float part[2][NW][NAX_WAVE * NCH];
   __shared__ double red[NW];
   __shared__ double shift[NW];
   int c = blockIdx.x;
@@ -206,14 +310,17 @@ __global__ __launch_bounds__(kEcsThreads, NCH <= 4 ? 4 : 2) void ecs_eval_kernel
   const int d = a.d, m = a.m;
   const float* zc = z + (int64_t)c * ldz;
   const int* idx = idx_all + (int64_t)c * m;
-  for (int k = threadIdx.x; k < kEcsMaxD; k += kEcsThreads) {
-    beta[k] = k < d ? zc[k] : 0.0f;
-    dlt[k] = (a.proxy && k < d) ? (double)zc[k] - a.bref[k] : 0.0;
-  }
-  __syncthreads();
-  const int wv = threadIdx.x / NAX_WAVE, ln = threadIdx.x % NAX_WAVE;
-  const int nch = (d + NAX_WAVE - 1) / NAX_WAVE;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / NAX_WAVE);
+  const int ln = threadIdx.x % NAX_WAVE, lr = ln % ROWS;
   const double nm = (double)a.n / m;
+  float beta[NCH];
+  int col[NCH];
+#pragma unroll
+  for (int t = 0; t < NCH; ++t) {
+    const int k = ln + t * NAX_WAVE;
+    beta[t] = k < d ? zc[k] : 0.0f;
+    col[t] = min(k, d - 1);
+  }
   // S1 and S2 - d0 S1 in fp32, d0 = the diff of this wave's first row (so
   // the final combination has no large cancelling terms)
   float s1[NCH], s2[NCH];
@@ -221,113 +328,119 @@ __global__ __launch_bounds__(kEcsThreads, NCH <= 4 ? 4 : 2) void ecs_eval_kernel
   for (int t = 0; t < NCH; ++t) s1[t] = s2[t] = 0.0f;
   double sd = 0, sd2 = 0;  // lanes 0..ROWS-1: sum diff, sum diff^2
   double d0 = 0.0;
-  auto load_rows = [&](int jb, float (&dst)[ROWS][NCH]) {
-    const float* xr[ROWS];
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) xr[r] = a.x + (int64_t)idx[min(jb + r, m - 1)] * d;
-#pragma unroll
-    for (int t = 0; t < NCH; ++t) {
-      const int k = ln + t * NAX_WAVE;
-      const bool ok = t < nch && k < d;
-#pragma unroll
-      for (int r = 0; r < ROWS; ++r) dst[r][t] = ok ? xr[r][k] : 0.0f;
-    }
+  // a step's rows j0 .. j0 + ROWS - 1: lane r holds the index and the record of
+  // row r; rows past m are zeros
+  struct Step {
+    float x[ROWS][NCH];
+    EcsRow q;
+    float y;
   };
-  float xv[ROWS][NCH];
-  int j0 = wv * ROWS;
-  if (j0 < m) load_rows(j0, xv);
-  for (bool first = true; j0 < m; j0 += NW * ROWS, first = false) {
-    // the next step's rows are in flight while this step is reduced
-    float xn[ROWS][NCH];
-    const int jn = j0 + NW * ROWS;
-    if (jn < m) load_rows(jn, xn);
-    float s[ROWS];
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) s[r] = 0.0f;
-#pragma unroll
-    for (int t = 0; t < NCH; ++t) {
-      const int k = ln + t * NAX_WAVE;
-      const float b = (t < nch && k < d) ? beta[k] : 0.0f;
-#pragma unroll
-      for (int r = 0; r < ROWS; ++r) s[r] = fmaf(xv[r][t], b, s[r]);
-    }
-    float mine = 0.0f;
+  auto load_idx = [&](int j0) { return idx[min(j0 + lr, m - 1)]; };
+  auto load_rows = [&](int j0, int iv, Step& st) {
+    if (a.proxy) st.q = a.rows[iv];
+    else st.y = a.y[iv];
+    const bool all = j0 + ROWS <= m;
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
-      const float t = wave_sum(s[r]);
-      if (ln == r) mine = t;
-    }
-    const int j = j0 + ln;
-    double df = 0, cc = 0;
-    if (ln < ROWS && j < m) {
-      const int64_t i = idx[j];
-      const double l = mine;
-      if (a.proxy) {
-        const EcsRow q = a.rows[i];
-        const double y = ecs_y(q), w = ecs_w(q);
-        const double dl = l - q.l_ref;
-        double ll, dy;
-        bern_terms(l, y, ll, dy);
-        df = ll - (q.ll_ref + q.r * dl - 0.5 * w * dl * dl);
-        cc = dy - q.r + w * dl;
+      const float* xr = a.x + (int64_t)__builtin_amdgcn_readlane(iv, r) * d;
+      if (all || j0 + r < m) {
+#pragma unroll
+        for (int t = 0; t < NCH; ++t) st.x[r][t] = xr[col[t]];
       } else {
-        double dy;
-        bern_terms(l, a.y[i], df, dy);
-        cc = nm * dy;
+#pragma unroll
+        for (int t = 0; t < NCH; ++t) st.x[r][t] = 0.0f;
       }
+    }
+  };
+  auto use_rows = [&](int j0, bool first, Step& st) {
+    // columns past d (the last chunks' lanes) read a column of the row again
+#pragma unroll
+    for (int t = NCH > 4 ? 4 : NCH - 1; t < NCH; ++t)
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) st.x[r][t] = ln + t * NAX_WAVE < d ? st.x[r][t] : 0.0f;
+    float s[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      s[r] = 0.0f;
+#pragma unroll
+      for (int t = 0; t < NCH; ++t) s[r] = fmaf(st.x[r][t], beta[t], s[r]);
+    }
+    const double l = rows_sum<ROWS>(s, ln);
+    double df, cc;
+    if (a.proxy) {
+      const double y = ecs_y(st.q), w = ecs_w(st.q);
+      const double dl = l - st.q.l_ref;
+      double ll, dy;
+      bern_terms(l, y, ll, dy);
+      df = ll - (st.q.ll_ref + st.q.r * dl - 0.5 * w * dl * dl);
+      cc = dy - st.q.r + w * dl;
+    } else {
+      double dy;
+      bern_terms(l, st.y, df, dy);
+      cc = nm * dy;
+    }
+    if (j0 + lr >= m) df = cc = 0.0;
+    if (ln < ROWS) {
       sd += df;
       sd2 += df * df;
     }
-    if (first) d0 = __shfl(df, 0, NAX_WAVE);
+    if (first) d0 = read_lane(df, 0);
     const float ccf = (float)cc, dcf = (float)((df - d0) * cc);
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
-      const float cr = __shfl(ccf, r, NAX_WAVE);
-      const float dcr = __shfl(dcf, r, NAX_WAVE);
+      const float cr = read_lane(ccf, r), dcr = read_lane(dcf, r);
 #pragma unroll
       for (int t = 0; t < NCH; ++t) {
-        s1[t] = fmaf(cr, xv[r][t], s1[t]);
-        s2[t] = fmaf(dcr, xv[r][t], s2[t]);
+        s1[t] = fmaf(cr, st.x[r][t], s1[t]);
+        s2[t] = fmaf(dcr, st.x[r][t], s2[t]);
       }
     }
-    if (jn < m) {
-#pragma unroll
-      for (int r = 0; r < ROWS; ++r)
-#pragma unroll
-        for (int t = 0; t < NCH; ++t) xv[r][t] = xn[r][t];
+  };
+  constexpr int STEP = NW * ROWS;
+  int j0 = wv * ROWS;
+  if (j0 < m) {
+    Step sa, sb;
+    load_rows(j0, load_idx(j0), sa);
+    int iv = load_idx(j0 + STEP);
+    for (bool first = true;; first = false) {
+      const bool more = j0 + STEP < m;
+      if (more) load_rows(j0 + STEP, iv, sb);
+      iv = load_idx(j0 + 2 * STEP);
+      use_rows(j0, first, sa);
+      if (!more) break;
+      j0 += STEP;
+      const bool more2 = j0 + STEP < m;
+      if (more2) load_rows(j0 + STEP, iv, sa);
+      iv = load_idx(j0 + 2 * STEP);
+      use_rows(j0, false, sb);
+      if (!more2) break;
+      j0 += STEP;
     }
   }
 #pragma unroll
   for (int t = 0; t < NCH; ++t) {
-    const int k = ln + t * NAX_WAVE;
-    if (t < nch && k < d) {
-      part[0][wv][k] = s1[t];
-      part[1][wv][k] = s2[t];
-    }
+    part[0][wv][ln + t * NAX_WAVE] = s1[t];
+    part[1][wv][ln + t * NAX_WAVE] = s2[t];
   }
   if (ln == 0) shift[wv] = d0;
-  // (H delta)_k for this thread's coordinates k = tid + 256 q, kept for the
-  // gradient; H is symmetric, so column reads are coalesced
-  double hk[kEcsMaxD / kEcsThreads];
-#pragma unroll
-  for (int q = 0; q < kEcsMaxD / kEcsThreads; ++q) {
-    hk[q] = 0.0;
-    const int k = threadIdx.x + q * kEcsThreads;
-    if (a.proxy && k < d)
-      for (int l2 = 0; l2 < d; ++l2) hk[q] += a.H[(int64_t)l2 * d + k] * dlt[l2];
-  }
-  const double mean = block_sum(sd, red) / m;  // block_sum synchronises first
-  double est, w1, w2;
+  const double mean = block_sum<NW>(sd, red) / m;  // block_sum synchronises first
+  const double* hc = hd + (int64_t)c * d;
+  double est, w1, w2, h1 = 0.0;
   if (a.proxy) {
-    const double var = fmax(block_sum(sd2, red) / m - mean * mean, 0.0);
-    // full-data proxy: LL + G.delta + delta.H delta / 2
-    double gd = 0;
-#pragma unroll
-    for (int q = 0; q < kEcsMaxD / kEcsThreads; ++q) {
-      const int k = threadIdx.x + q * kEcsThreads;
-      if (k < d) gd += dlt[k] * (a.G[k] + 0.5 * hk[q]);
+    const double var = fmax(block_sum<NW>(sd2, red) / m - mean * mean, 0.0);
+    // full-data proxy: LL + G.delta + delta.H delta / 2; H = 0 for degree 1,
+    // where H delta is 0, or NaN if delta is not finite
+    double gd = 0, sx = 0;
+    for (int k = threadIdx.x; k < d; k += NT) {
+      const double dk = (double)zc[k] - a.bref[k];
+      gd += dk * (a.G[k] + (a.proxy == 2 ? 0.5 * hc[k] : 0.0));
+      sx += dk;
     }
-    const double full = a.LL + block_sum(gd, red);
+    if (a.proxy != 2) {
+      h1 = 0.0 * block_sum<NW>(sx, red);
+      gd += h1;
+    }
+    const double full = a.LL + block_sum<NW>(gd, red);
     est = full + (double)a.n * mean - 0.5 * (double)a.n * nm * var;
     w1 = nm * (1.0 + nm * mean);
     w2 = nm * nm;
@@ -340,24 +453,20 @@ __global__ __launch_bounds__(kEcsThreads, NCH <= 4 ? 4 : 2) void ecs_eval_kernel
   const double s2v = a.prior_scale * a.prior_scale;
   const double cst = log(a.prior_scale) + 0.91893853320467274178;  // log s + log(2 pi) / 2
   double pr = 0;
-  for (int k = threadIdx.x; k < d; k += kEcsThreads)
-    pr += 0.5 * (double)beta[k] * beta[k] / s2v + cst;
-  pr = block_sum(pr, red);  // also orders the part[] writes before the reads below
+  for (int k = threadIdx.x; k < d; k += NT) pr += 0.5 * (double)zc[k] * zc[k] / s2v + cst;
+  pr = block_sum<NW>(pr, red);  // also orders the part[] writes before the reads below
   if (threadIdx.x == 0) pe[c] = pr - est;
+  for (int k = threadIdx.x; k < d; k += NT) {
+    double t1 = 0, t2 = 0;
 #pragma unroll
-  for (int q = 0; q < kEcsMaxD / kEcsThreads; ++q) {
-    const int k = threadIdx.x + q * kEcsThreads;
-    if (k < d) {
-      double t1 = 0, t2 = 0;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        t1 += part[0][w][k];
-        t2 += part[1][w][k] + shift[w] * part[0][w][k];
-      }
-      double acc = w1 * t1 - w2 * t2;
-      if (a.proxy) acc += a.G[k] + hk[q];
-      g[(int64_t)c * ldg + k] = (float)((double)beta[k] / s2v - acc);
+    for (int w = 0; w < NW; ++w) {
+      const double p0 = part[0][w][k];
+      t1 += p0;
+      t2 += (double)part[1][w][k] + shift[w] * p0;
     }
+    double acc = w1 * t1 - w2 * t2;
+    if (a.proxy) acc += a.G[k] + (a.proxy == 2 ? hc[k] : h1);
+    g[(int64_t)c * ldg + k] = (float)((double)zc[k] / s2v - acc);
   }
 }
 
@@ -458,11 +567,14 @@ struct EcsLogistic : Potential {
   double* pe_new = nullptr;
   float* g_new = nullptr;
   double* buf = nullptr;  // bref, per-row scalars, G, H
+  double* hd = nullptr;   // H delta of each chain [hd_chains][d], degree 2
+  int hd_chains = 0;
   ~EcsLogistic() override {
     (void)hipFree(prop);
     (void)hipFree(pe_new);
     (void)hipFree(g_new);
     (void)hipFree(buf);
+    (void)hipFree(hd);
   }
   int dim() const override { return a.d; }
   const char* name() const override { return "ecs_eval_kernel"; }
@@ -475,16 +587,44 @@ struct EcsLogistic : Potential {
   double alg_flops(int C_) const override { return 4.0 * C_ * a.m * a.d; }
   hipError_t launch(hipStream_t s, const int* ix, const float* z, int ldz, int grid, const int* act,
                     const int* nact, double* pe, float* g, int ldg, bool mark = true) {
+    if (a.proxy == 2) {
+      if (grid > hd_chains) {
+        (void)hipFree(hd);
+        hd = nullptr;
+        hd_chains = 0;
+        const hipError_t e = hipMalloc(&hd, sizeof(double) * (size_t)grid * a.d);
+        if (e != hipSuccess) return e;
+        hd_chains = grid;
+      }
+      hipLaunchKernelGGL(ecs_proxy_kernel, dim3((grid + kProxyChains - 1) / kProxyChains),
+                         dim3(kEcsThreads * kProxyParts), 0, s, a, z, ldz, grid, act, nact, hd);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
     if (mark) mark_begin(s);
-    const dim3 gr(grid), bl(kEcsThreads);
+    // Up to 256 chains (the CUs) a chain's rows go to eight waves, else to four,
+    // with two workgroups per CU: m = 1000, d = 256, 256 chains on eight waves 64 us
+    // with the proxy's kernel, 257 on four 78.
+#define NAX_ECS_NW(NCHV, RV, NWV)                                                             \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(ecs_eval_kernel<NCHV, RV, NWV>), dim3(grid),                \
+                     dim3(NWV * NAX_WAVE), 0, s, a, ix, z, ldz, hd, act, nact, pe, g, ldg)
+#define NAX_ECS(NCHV, RV)                            \
+  do {                                               \
+    if (grid <= 256) NAX_ECS_NW(NCHV, RV, 8);        \
+    else NAX_ECS_NW(NCHV, RV, 4);                    \
+  } while (0)
     if (a.d <= 64)
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(ecs_eval_kernel<1, 8>), gr, bl, 0, s, a, ix, z, ldz, act, nact, pe, g, ldg);
+      NAX_ECS(1, 16);
     else if (a.d <= 128)
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(ecs_eval_kernel<2, 8>), gr, bl, 0, s, a, ix, z, ldz, act, nact, pe, g, ldg);
+      NAX_ECS(2, 16);
+    else if (a.d <= 192)
+      NAX_ECS(3, 16);
     else if (a.d <= 256)
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(ecs_eval_kernel<4, 4>), gr, bl, 0, s, a, ix, z, ldz, act, nact, pe, g, ldg);
+      NAX_ECS(4, 16);
     else
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(ecs_eval_kernel<8, 2>), gr, bl, 0, s, a, ix, z, ldz, act, nact, pe, g, ldg);
+      NAX_ECS(8, 8);
+#undef NAX_ECS
+#undef NAX_ECS_NW
     if (mark) mark_end(s);
     return hipGetLastError();
   }
@@ -541,6 +681,10 @@ Potential* make_ecs_logistic(const float* x, const float* y, int64_t n, int d, d
   if ((e = hipMalloc(&p->pe_new, sizeof(double) * num_chains))) return fail("hipMalloc", e);
   if ((e = hipMalloc(&p->g_new, sizeof(float) * (size_t)num_chains * Dp))) return fail("hipMalloc", e);
   if (!proxy) return p;
+  if (proxy == 2) {
+    if ((e = hipMalloc(&p->hd, sizeof(double) * (size_t)num_chains * d))) return fail("hipMalloc", e);
+    p->hd_chains = num_chains;
+  }
   // [rows: n records of 4 doubles][bref d][G d][H d*d]
   const size_t nbuf = 4 * (size_t)n + d + d + (size_t)d * d;
   if ((e = hipMalloc(&p->buf, sizeof(double) * nbuf))) return fail("hipMalloc", e);
