@@ -161,6 +161,31 @@ __device__ __forceinline__ double chain_inclusive_scan(const G& g, double v) {
   return v;
 }
 
+// chain_sum(v) in `total` and chain_inclusive_scan(v), the same values, with the
+// waves' parts of both exchanged at one pair of barriers.
+template <class G>
+__device__ __forceinline__ double chain_sum_and_scan(const G& g, double v, double& total) {
+  const double s = wave_sum(v);
+  v = wave_inclusive_scan(v, g.lane & (NAX_WAVE - 1));
+  total = s;
+  if constexpr (G::WPC > 1) {
+    const int w = g.lane / NAX_WAVE;
+    __syncthreads();
+    if ((g.lane & (NAX_WAVE - 1)) == NAX_WAVE - 1) {
+      g.red[w] = v;
+      g.red[G::WPC + w] = s;
+    }
+    __syncthreads();
+    double off = 0.0, t = 0.0;
+    for (int k = 0; k < w; ++k) off += g.red[k];
+#pragma unroll
+    for (int k = 0; k < G::WPC; ++k) t += g.red[G::WPC + k];
+    v += off;
+    total = t;
+  }
+  return v;
+}
+
 // The group a standalone (non-persistent) evaluation of one chain runs on:
 // one wavefront.
 struct WaveGroup {
