@@ -77,6 +77,10 @@ struct ChainCtxT {
   // FOR_D's unroll: the translation unit's factor for one wave, divided by
   // the waves (each thread walks WPC times fewer elements)
   static constexpr int UNROLL = NAX_FOR_D_UNROLL / WPC_ > 0 ? NAX_FOR_D_UNROLL / WPC_ : 1;
+  // Elements of a thread that the leaf's passes load before they store any: a
+  // pass that stores an element first waits for every load of the next one, as
+  // the slots may alias for all the compiler knows.
+  static constexpr int BATCH = NAX_FOR_D_UNROLL > 1 ? 4 : 1;
   double* red;     // LDS reduction slots of the group (kRedSlots * WPC), WPC > 1
   float* redf;     // LDS [WPC][64] fp32 exchange of the group, WPC > 1
   float* vb;       // chain's vector block [nvec][Dp]
@@ -92,6 +96,11 @@ struct ChainCtxT {
     if constexpr (LDSV) return (slot < V_HOT ? lb : vb) + (size_t)slot * Dp;
     return vb + (size_t)slot * Dp;
   }
+  // A slot below V_HOT / from V_HOT on, where the slot is a run-time value: the
+  // address space is known, so that its accesses are LDS or global ones and not
+  // flat.
+  __device__ float* hot(int slot) const { return (LDSV ? lb : vb) + (size_t)slot * Dp; }
+  __device__ float* cold(int slot) const { return vb + (size_t)slot * Dp; }
 };
 using ChainCtx = ChainCtxT<false>;
 
@@ -211,11 +220,23 @@ __device__ __forceinline__ float dense_mv(const CX& cx, const float* at, const f
   return a0 + a1;
 }
 
+// a[0 .. D) = b[0 .. D), BATCH loads of a thread in flight.
+template <class CX>
+__device__ __forceinline__ void copy_slot(const CX& cx, float* a, const float* b) {
+  constexpr int B = CX::BATCH;
+  for (int d0 = cx.lane; d0 < cx.D; d0 += B * CX::NT) {
+    float x[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) x[j] = b[j == 0 ? d0 : min(d0 + j * CX::NT, cx.D - 1)];
+#pragma unroll
+    for (int j = 0; j < B; ++j)
+      if (j == 0 || d0 + j * CX::NT < cx.D) a[d0 + j * CX::NT] = x[j];
+  }
+}
+
 template <class CX>
 __device__ __forceinline__ void vcopy(const CX& cx, int dst, int src) {
-  float* a = cx.v(dst);
-  const float* b = cx.v(src);
-  FOR_D(d) a[d] = b[d];
+  copy_slot(cx, cx.v(dst), cx.v(src));
 }
 
 // euclidean_kinetic_energy (hmc_util.py:1183-1200): 0.5 r . (M^-1 r)
@@ -284,9 +305,9 @@ __device__ __forceinline__ void draw_momentum(const CX& cx, int dst, Key k, bool
 template <class CX>
 __device__ __forceinline__ void leapfrog_half(const CX& cx, int zs, int rs, int gs, float eps,
                               float* zreq) {
-  float* z = cx.v(zs);
-  float* r = cx.v(rs);
-  const float* g = cx.v(gs);
+  float* z = cx.hot(zs);
+  float* r = cx.hot(rs);
+  const float* g = cx.hot(gs);
   const float* m = cx.v(V_IMM);
   const float h = 0.5f * eps;
   if (cx.mi) {
@@ -299,12 +320,28 @@ __device__ __forceinline__ void leapfrog_half(const CX& cx, int zs, int rs, int 
     }
     return;
   }
-  FOR_D(d) {
-    float rh = r[d] - h * g[d];
-    float zn = z[d] + eps * (m[d] * rh);
-    r[d] = rh;
-    z[d] = zn;
-    if (zreq) zreq[d] = zn;
+  constexpr int B = CX::BATCH;
+  for (int d0 = cx.lane; d0 < cx.D; d0 += B * CX::NT) {
+    float rv[B], gv[B], zv[B], mv[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      const int d = j == 0 ? d0 : min(d0 + j * CX::NT, cx.D - 1);
+      rv[j] = r[d];
+      gv[j] = g[d];
+      zv[j] = z[d];
+      mv[j] = m[d];
+    }
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      const float rh = rv[j] - h * gv[j];
+      const float zn = zv[j] + eps * (mv[j] * rh);
+      const int d = d0 + j * CX::NT;
+      if (j == 0 || d < cx.D) {
+        r[d] = rh;
+        z[d] = zn;
+        if (zreq) zreq[d] = zn;
+      }
+    }
   }
 }
 
@@ -312,8 +349,8 @@ __device__ __forceinline__ void leapfrog_half(const CX& cx, int zs, int rs, int 
 template <class CX>
 __device__ __forceinline__ void leapfrog_finish(const CX& cx, int rs, int gs, float eps,
                                 const float* gin) {
-  float* r = cx.v(rs);
-  float* g = cx.v(gs);
+  float* r = cx.hot(rs);
+  float* g = cx.hot(gs);
   const float h = 0.5f * eps;
   FOR_D(d) {
     float gv = gin[d];
@@ -339,37 +376,62 @@ __device__ __forceinline__ void leaf_pass(const CX& cx, int rs, int gs, float ep
                                           double (&out)[1 + 2 * NCHK]) {
   const float* ckr[3] = {ckr0, ckr1, ckr2};
   const float* cks[3] = {cks0, cks1, cks2};
-  float* r = cx.v(rs);
-  float* g = cx.v(gs);
+  float* r = cx.hot(rs);
+  float* g = cx.hot(gs);
   float* srs = cx.v(V_SRSUM);
   const float* m = cx.v(V_IMM);
   const float h = 0.5f * eps;
+  constexpr int NQ = NCHK > 0 ? NCHK : 1, B = CX::BATCH;
   double acc = 0.0;
-  double a[NCHK > 0 ? NCHK : 1], b[NCHK > 0 ? NCHK : 1];
+  double a[NQ], b[NQ];
 #pragma unroll
-  for (int j = 0; j < NCHK; ++j) a[j] = b[j] = 0.0;
-  FOR_D(d) {
-    const float gv = gin[d];
-    g[d] = gv;
-    const float rv = r[d] - h * gv;
-    r[d] = rv;
-    const double rd = rv;
-    acc += (double)m[d] * rd * rd;
-    const float s = first ? rv : srs[d] + rv;
-    srs[d] = s;
-    if constexpr (NCHK == 0) {
-      ckr_w[d] = rv;
-      cks_w[d] = s;
+  for (int q = 0; q < NCHK; ++q) a[q] = b[q] = 0.0;
+  for (int d0 = cx.lane; d0 < cx.D; d0 += B * CX::NT) {
+    float gv[B], rv[B], mv[B], sv[B], rl[B][NQ], sl[B][NQ];
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      const int d = j == 0 ? d0 : min(d0 + j * CX::NT, cx.D - 1);
+      gv[j] = gin[d];
+      rv[j] = r[d];
+      mv[j] = m[d];
+      sv[j] = srs[d];
+#pragma unroll
+      for (int q = 0; q < NCHK; ++q) {
+        rl[j][q] = ckr[q][d];
+        sl[j][q] = cks[q][d];
+      }
     }
 #pragma unroll
-    for (int j = 0; j < NCHK; ++j) {
-      const float rlv = ckr[j][d];
-      const float sj = s - cks[j][d] + rlv;
-      const float c = sj - (rlv + rv) * 0.5f;
-      const float vl = m[d] * rlv;
-      const float vr = m[d] * rv;
-      a[j] += (double)vl * c;
-      b[j] += (double)vr * c;
+    for (int j = 0; j < B; ++j) {
+      const bool in = j == 0 || d0 + j * CX::NT < cx.D;
+      rv[j] = rv[j] - h * gv[j];
+      const double rd = rv[j];
+      const double t = acc + (double)mv[j] * rd * rd;
+      acc = in ? t : acc;
+      sv[j] = first ? rv[j] : sv[j] + rv[j];
+#pragma unroll
+      for (int q = 0; q < NCHK; ++q) {
+        const float sj = sv[j] - sl[j][q] + rl[j][q];
+        const float c = sj - (rl[j][q] + rv[j]) * 0.5f;
+        const float vl = mv[j] * rl[j][q];
+        const float vr = mv[j] * rv[j];
+        const double ta = a[q] + (double)vl * c, tb = b[q] + (double)vr * c;
+        a[q] = in ? ta : a[q];
+        b[q] = in ? tb : b[q];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      const int d = d0 + j * CX::NT;
+      if (j == 0 || d < cx.D) {
+        g[d] = gv[j];
+        r[d] = rv[j];
+        srs[d] = sv[j];
+        if constexpr (NCHK == 0) {
+          ckr_w[d] = rv[j];
+          cks_w[d] = sv[j];
+        }
+      }
     }
   }
   out[0] = acc;
@@ -758,9 +820,9 @@ __device__ __forceinline__ bool advance_chain(const EngineCfg& cfg, const Collec
         const int nsub = __popc((unsigned)((~leaf_idx & (leaf_idx + 1)) - 1));
         const int idx_min = idx_max - nsub + 1;
         const bool even = (leaf_idx & 1) == 0;  // even: writes checkpoint idx_max, no checks
-        const float* znew = cx.v(zs);
-        const float* rnew = cx.v(rs);
-        const float* gnew = cx.v(gs);
+        const float* znew = cx.hot(zs);
+        const float* rnew = cx.hot(rs);
+        const float* gnew = cx.hot(gs);
         float* srs = cx.v(V_SRSUM);
         double kin;
         bool turning = false;
@@ -770,22 +832,22 @@ __device__ __forceinline__ bool advance_chain(const EngineCfg& cfg, const Collec
           kin = kinetic(cx, rs);
           FOR_D(d) srs[d] = leaf_idx == 0 ? rnew[d] : srs[d] + rnew[d];
           if (even) {
-            float* ckr = cx.v(CKR + idx_max);
-            float* cks = cx.v(CKS + idx_max);
+            float* ckr = cx.cold(CKR + idx_max);
+            float* cks = cx.cold(CKS + idx_max);
             FOR_D(d) { ckr[d] = rnew[d]; cks[d] = srs[d]; }
           }
         } else {  // the same values from one pass and one reduction
           const int nf = even ? 0 : (nsub < 3 ? nsub : 3);
           // checkpoints idx_max, idx_max - 1, idx_max - 2 (those beyond nf unused)
           const int i1 = nf > 1 ? idx_max - 1 : idx_max, i2 = nf > 2 ? idx_max - 2 : idx_max;
-          const float* r0 = cx.v(CKR + idx_max);
-          const float* s0 = cx.v(CKS + idx_max);
-          const float* r1 = cx.v(CKR + i1);
-          const float* s1 = cx.v(CKS + i1);
-          const float* r2 = cx.v(CKR + i2);
-          const float* s2 = cx.v(CKS + i2);
-          float* ckr_w = even ? cx.v(CKR + idx_max) : nullptr;
-          float* cks_w = even ? cx.v(CKS + idx_max) : nullptr;
+          const float* r0 = cx.cold(CKR + idx_max);
+          const float* s0 = cx.cold(CKS + idx_max);
+          const float* r1 = cx.cold(CKR + i1);
+          const float* s1 = cx.cold(CKS + i1);
+          const float* r2 = cx.cold(CKR + i2);
+          const float* s2 = cx.cold(CKS + i2);
+          float* ckr_w = even ? cx.cold(CKR + idx_max) : nullptr;
+          float* cks_w = even ? cx.cold(CKS + idx_max) : nullptr;
           const bool first = leaf_idx == 0;
           // _is_turning's verdict for checkpoint j of the pass: either sum <= 0
           auto turn = [](const double* o, int j) {
@@ -827,7 +889,7 @@ __device__ __forceinline__ bool advance_chain(const EngineCfg& cfg, const Collec
           next_check = idx_max - nf;
         }
         for (int i = next_check; i >= idx_min && !turning; --i)
-          turning = is_turning(cx, cx.v(CKR + i), rnew, srs, cx.v(CKS + i), cx.v(CKR + i));
+          turning = is_turning(cx, cx.cold(CKR + i), rnew, srs, cx.cold(CKS + i), cx.cold(CKR + i));
         const double pe_new = pe_in;
         const double e_new = pe_new + kin;
         const double delta = nan_to_inf(e_new - S.energy_current);
@@ -837,7 +899,8 @@ __device__ __forceinline__ bool advance_chain(const EngineCfg& cfg, const Collec
         float* szp = cx.v(V_SZP);
         float* sgp = cx.v(V_SGP);
         if (leaf_idx == 0) {
-          FOR_D(d) { szp[d] = znew[d]; sgp[d] = gnew[d]; }
+          copy_slot(cx, szp, znew);
+          copy_slot(cx, sgp, gnew);
           S.s_peP = pe_new; S.s_energyP = e_new; S.s_weight = leaf_w;
           S.s_diverging = leaf_div; S.s_sum_accept = acc; S.s_num = 1;
         } else {  // _combine_tree(..., biased_transition=False) (hmc_util.py:767-848)
@@ -845,7 +908,8 @@ __device__ __forceinline__ bool advance_chain(const EngineCfg& cfg, const Collec
           const double e = exp(-fabs(x));
           const double p = expit_e(x, e);
           if (bernoulli(K(S.leaf_key), p, part)) {
-            FOR_D(d) { szp[d] = znew[d]; sgp[d] = gnew[d]; }
+            copy_slot(cx, szp, znew);
+            copy_slot(cx, sgp, gnew);
             S.s_peP = pe_new; S.s_energyP = e_new;
           }
           S.s_weight = log_add_exp_e(S.s_weight, leaf_w, e);
@@ -964,6 +1028,19 @@ __device__ __forceinline__ void request_slots(const ChainState& S, int& zs, int&
   const bool left = S.phase == PH_LEAF_WAIT && !S.going_right;
   zs = left ? V_ZL : V_ZR;
   gs = left ? V_GL : V_GR;
+}
+
+// The gradient a chain waits for at the start of a launch, moved from the host's
+// buffer to the slot its phase reads later ones from, so that all are LDS reads.
+template <class CX>
+__device__ __forceinline__ const float* gradient_to_slot(const CX& cx, const ChainState& S,
+                                                         const float* gi) {
+  int zs, gs;
+  request_slots(S, zs, gs);
+  float* gh = cx.hot(gs);
+  if (S.phase != PH_ITER_START) FOR_D(d) gh[d] = gi[d];
+  chain_sync(cx);
+  return gh;
 }
 
 // Chain index of the calling wavefront (`wpb` wavefronts per block), made
@@ -1135,15 +1212,16 @@ persistent_kernel(M m, EngineCfg cfg, Collect col, const int64_t* __restrict__ d
   const int wave_lane = threadIdx.x & (NAX_WAVE - 1);
   ChainState& S = sS[threadIdx.x / NAX_WAVE];
   copy_state(S, states[c], wave_lane);
+  if constexpr (LDSV) gi = gradient_to_slot(cx, S, gi);
   double pe = peout[c];
   int evals = 0;
   while (advance_chain(cfg, col, target, S, cx, c, nullptr, gi, pe, evals)) {
     int zs, gs;
     request_slots(S, zs, gs);
     chain_sync(cx);
-    pe = m.value_and_grad(cx, cx.v(zs), cx.v(gs));
+    pe = m.value_and_grad(cx, cx.hot(zs), cx.hot(gs));
     chain_sync(cx);
-    gi = cx.v(gs);
+    gi = cx.hot(gs);
   }
   if constexpr (LDSV) {
     __syncthreads();
@@ -1194,7 +1272,10 @@ persistent_head_kernel(M m, EngineCfg cfg, Collect col, const int64_t* __restric
   }
   // the first call may take a gradient the host evaluated (initialisation)
   const float* gi = gout + (size_t)c * cfg.Dp;
-  if (head) copy_state(sS, states[c], hx.lane);
+  if (head) {
+    copy_state(sS, states[c], hx.lane);
+    if constexpr (LDSV) gi = gradient_to_slot(hx, sS, gi);
+  }
   double pe = peout[c];
   int evals = 0;
   for (;;) {
@@ -1211,9 +1292,9 @@ persistent_head_kernel(M m, EngineCfg cfg, Collect col, const int64_t* __restric
     __syncthreads();
     const int more = req[0], zs = req[1], gs = req[2];
     if (!more) break;
-    pe = m.value_and_grad(gx, gx.v(zs), gx.v(gs));
+    pe = m.value_and_grad(gx, gx.hot(zs), gx.hot(gs));
     __syncthreads();  // the gradient is written, req has been read
-    gi = gx.v(gs);
+    gi = gx.hot(gs);
   }
   if constexpr (LDSV) {
     const int n = nl * cfg.Dp;
