@@ -534,8 +534,7 @@ class HMC(MCMCKernel):
         if z0.ndim <= 1 and num_chains == 1:
             z0 = z0.reshape(1, -1)
         model = _as_model(target, z0[0] if z0.ndim > 1 else z0)
-        init_keys = np.stack([nrandom.split(k)[0] for k in keys]) if num_chains <= 8 else \
-            _split_first(keys)
+        init_keys = _split_at(np.asarray(keys, dtype=np.uint32).reshape(-1, 2), 0)
         eng = Engine(model, num_chains, self._algo, num_warmup, step_size=self._step_size,
                      adapt_step_size=self._adapt_step_size,
                      adapt_mass_matrix=self._adapt_mass_matrix, dense_mass=self._dense_mass,
@@ -598,14 +597,6 @@ class NUTS(HMC):
                          init_strategy=init_strategy)
         self._max_tree_depth = max_tree_depth
         self._algo = "NUTS"
-
-
-def _split_first(keys):
-    """split(k)[0] for each key, on the device."""
-    out = np.empty_like(keys)
-    for c in range(keys.shape[0]):
-        out[c] = nrandom.split(keys[c])[0]
-    return out
 
 
 def _site_layout(model):
