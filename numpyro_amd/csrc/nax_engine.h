@@ -79,7 +79,8 @@ struct ChainCtxT {
   static constexpr int UNROLL = NAX_FOR_D_UNROLL / WPC_ > 0 ? NAX_FOR_D_UNROLL / WPC_ : 1;
   // Elements of a thread that the leaf's passes load before they store any: a
   // pass that stores an element first waits for every load of the next one, as
-  // the slots may alias for all the compiler knows.
+  // the slots may alias for all the compiler knows (T = 3000 on 4 waves, one chain:
+  // 15.9 -> 14.4 us per leaf, with hot() and cold() below).
   static constexpr int BATCH = NAX_FOR_D_UNROLL > 1 ? 4 : 1;
   double* red;     // LDS reduction slots of the group (kRedSlots * WPC), WPC > 1
   float* redf;     // LDS [WPC][64] fp32 exchange of the group, WPC > 1
