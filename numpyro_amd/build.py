@@ -22,6 +22,11 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
 ]
+# logistic_split: its wide kernels use more than 256 registers and add to their
+# accumulators outside the MFMAs; left to itself the compiler keeps those in the
+# accumulation registers and copies them out and back around every addition
+# (500,000 x 250 in fp8, 250 chains: 960 us, 914 with the flag)
+FILE_FLAGS = {"logistic_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _run(cmd, what):
@@ -35,7 +40,7 @@ def _run(cmd, what):
 def build(verbose=False, jobs=None):
     os.makedirs(OBJ, exist_ok=True)
     objs = [os.path.join(OBJ, os.path.splitext(s)[0] + ".o") for s in SOURCES]
-    cmds = [[HIPCC] + FLAGS + ["-c", os.path.join(CSRC, s), "-o", o]
+    cmds = [[HIPCC] + FLAGS + FILE_FLAGS.get(s, []) + ["-c", os.path.join(CSRC, s), "-o", o]
             for s, o in zip(SOURCES, objs)]
     if verbose:
         for c in cmds:

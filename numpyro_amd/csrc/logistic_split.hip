@@ -9,23 +9,34 @@
 //
 // GEMM1 runs on the fp32 MFMA, whose accumulation is the chain of fp32 fused
 // multiply-adds over d = 0, 1, ... (v_mfma_f32_32x32x2_f32 against fmaf on
-// 200,000 random triples: every one equal): logits, and with them energies,
-// are those of the VALU tile kernel bit for bit.  A design in fp8 codes
-// enters as its code values (exact), its power-of-two column scales go to z.
+// 200,000 random triples: every one equal): logits are those of the VALU tile
+// kernel bit for bit.  (Energies are not: the fp32 forms take a row's loss from
+// logit_terms and add a lane's 16 rows of a tile in fp32 before the compensated
+// fp64 sum, fp8 takes log1p_unit and adds every row in fp64.)  A design in fp8
+// codes enters as its code values (exact), its power-of-two column scales go to z.
 //
-// GEMM2 runs on the fp16 MFMA, which takes 1/16 of the time: each fp32 factor
-// is a sum of two fp16 terms, hi = fp16(v) and lo = fp16(v - hi), and a product
-// is hi hi + hi lo + lo hi, three MFMAs with exact products and fp32
-// accumulation (fp8 codes are exact in one term: two MFMAs).  hi + lo keeps 22
-// to 23 bits of v, random in sign over the rows; the fp32 MFMA rounds its
-// accumulator every second row, this one every eighth.  The eight products
-// that the fp16 MFMA adds at once are cut (toward zero) 24 bits below the
-// largest, which would add up where r x is skewed; with hi on grids (R: 2^-10, X:
-// 2^-11 of the power of two above the column's rms) the hi hi products are
-// multiples of one step and nothing of them is cut.  Measured against
-// float64, gradient error relative to its norm, fp32 MFMA / split:
-// 200,000 x 100, 256 chains 6.8e-7 / 5.9e-7; 581,012 x 55, 256 chains 1.5e-6 /
-// 1.5e-6; 500,000 x 256, 1024 chains 2.9e-6 / 2.2e-6.
+// GEMM2 runs on the fp16 MFMA, which takes 1/16 of the time.  X' (the scaled
+// column) is two fp16 terms, hi + lo, and R' = 2^14 r three: a + (b + c) / 2^10.
+// hi and a lie on grids (X': 2^-11 of the power of two above the column's rms, R':
+// 2^-10 of |r| = 1), because the eight products that the fp16 MFMA adds at once
+// are cut (toward zero) 24 bits below the largest, which would add up where r x is
+// skewed: products a hi are multiples of one step, and nothing of them is cut.
+// b + c hold r - a to 22 bits of itself, for residuals down to 2^-26: with one term
+// below the grid a residual under 2^-11 (rare events) had 11 bits, and since
+// thousands of rows with the same covariates share it, their errors added up (error
+// of 1e-3 below).  The products with b and c are summed from zero over a tile and
+// added to the running sum once, so that they do not meet a large sum one by
+// one.  Five MFMAs a k-step (fp8 codes are exact in one term: three).  Gradient
+// error against float64 over the root of the sum of (r x)^2, rms over 256 chains
+// near the generating coefficients, both products on the fp32 MFMA / this / one
+// term below R's grid:
+//   581,012 x 55, covtype-like             2.3e-6 / 2.3e-6 / 2.3e-6
+//   500,000 x 250, normal                  1.4e-6 / 0.9e-6 / 1.3e-6
+//   1,000,000 rows in 8 categories, events at 1e-2   5.7e-5 / 6.9e-6 / 1.6e-4
+//                                              1e-3   5.2e-5 / 5.3e-6 / 3.4e-4
+//                                              1e-4   3.9e-5 / 2.0e-6 / 7.4e-4
+//   500,000 x 12 binary, intercept -7      2.3e-5 / 1.5e-6 / 1.8e-4
+//   the same, columns standardised         7.1e-5 / 6.8e-6 / 1.5e-4
 // (GEMM1 does not take the split: an error of z shifts every row's logit
 // alike, and near the mode the gradient answers to it sqrt(N) times over.)
 //
@@ -42,14 +53,15 @@
 // 2.0e-7 against 1.2e-7) and a launch is mostly latency.  Other designs take
 // the fp32 MFMA in GEMM2 too.
 //
-// Bound: MFMA issue (D = 256: GEMM1 8192 cycles per tile and wave, GEMM2 1536
+// Bound: MFMA issue (D = 256: GEMM1 8192 cycles per tile and wave, GEMM2 2560
 // split, 8192 in fp32) plus the epilogue's VALU work, which the fp32 MFMA hardly
 // overlaps (standing between the MFMAs or in groups of its own it takes the same
 // time); two blocks share a CU where the registers allow, so that one's GEMM2
-// runs beside the other's epilogue.  Main kernel, before (both products fp32,
-// epilogue between them) and now: 581,012 x 55, 256 chains 412 -> 281 us;
-// 2,000,000 x 256, 1024 chains (fp32 form) 17.0 -> 16.4 ms; fp8 500,000 x 250, 250
-// chains 13.6 ms (VALU tile kernel) -> 0.80.
+// runs beside the other's epilogue.  Main kernel, both products in fp32 and
+// split: 581,012 x 55, 256 chains 412 and 319 us (281 with one term below R's grid);
+// 500,000 x 250, 256 chains 1.06 and 0.85 ms (0.76); fp8 500,000 x 250, 250 chains
+// 13.6 ms on the VALU tile kernel and 0.90 (0.81).  2,000,000 x 256, 1024 chains
+// (fp32 form) 17.0 ms with the epilogue between the products, 16.5 as here.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -67,6 +79,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kRScale = 16384.0f;  // 2^14: |R'| <= 2^14
+constexpr float kRFine = 1024.0f;    // of the terms below R's grid
 constexpr int64_t kSplitRows = 32768, kSplitMin = 65536;
 
 // hi (on a grid of step q, a power of two, where fp16 is finer) + lo of a
@@ -260,8 +273,8 @@ __global__ void split_pad_y(const float* __restrict__ y, int64_t N, int64_t Np,
 
 // ---- the fused kernel ----------------------------------------------------------------
 
-// kSplitF32: fp32 design, GEMM2 by two fp16 terms; kPlainF32: GEMM2 on the fp32
-// MFMA; kSplitFp8: e4m3 codes, GEMM2 by two fp16 terms of R.
+// kSplitF32: fp32 design, GEMM2 by fp16 terms; kPlainF32: GEMM2 on the fp32
+// MFMA; kSplitFp8: e4m3 codes, GEMM2 by fp16 terms of R.
 enum { kSplitF32 = 0, kPlainF32 = 1, kSplitFp8 = 2 };
 
 // Bytes of a tile's GEMM1 part (A, fp32) and GEMM2 part (B) in LDS, and the slots
@@ -484,7 +497,7 @@ logit_split_kernel(const void* __restrict__ XA, const void* __restrict__ XB,
       f32x16 Ln;
 #pragma unroll
       for (int v = 0; v < 16; ++v) Ln[v] = 0.0f;
-      f16x8 rh[2], rl[2];
+      f16x8 ra[2], rm[2], rc[2];  // R' = ra + (rm + rc) / kRFine
       float rv[16];
       float us = 0.0f;
       f32x4 w = part(i + 1, 0);
@@ -515,10 +528,14 @@ logit_split_kernel(const void* __restrict__ XA, const void* __restrict__ XB,
         if constexpr (MODE == kPlainF32) {
           rv[e] = r;
         } else {
-          _Float16 a, b;
-          split16(r * kRScale, kRGrid, a, b);
-          rh[e / 8][e % 8] = a;
-          rl[e / 8][e % 8] = b;
+          const float v = r * kRScale;
+          constexpr float m = 12582912.0f * kRGrid;  // rounds to the grid
+          const float hi = (v + m) - m;
+          const float rest = (v - hi) * kRFine;  // exact
+          const _Float16 mid = (_Float16)rest;
+          ra[e / 8][e % 8] = (_Float16)hi;
+          rm[e / 8][e % 8] = mid;
+          rc[e / 8][e % 8] = (_Float16)(rest - (float)mid);
         }
         if (e < 15) __builtin_amdgcn_sched_barrier(0);
       }
@@ -547,15 +564,55 @@ logit_split_kernel(const void* __restrict__ XA, const void* __restrict__ XB,
             for (int j = 0; j < 4; ++j) g[dt] = mma32(rv[4 * m4 + j], b[j], g[dt]);
           }
       } else {
+        // column block dt: products of R's grid terms to g, of its fine terms to t
+        // from zero; after(k) follows product k
+        constexpr int NP = FP8 ? 6 : 10;
+        auto products = [&](int dt, f32x16& t, auto after) {
 #pragma unroll
-        for (int m2 = 0; m2 < 2; ++m2)
+          for (int v = 0; v < 16; ++v) t[v] = 0.0f;
+#pragma unroll
+          for (int m2 = 0; m2 < 2; ++m2) {
+            int k = m2 * (NP / 2);
+            const f16x8 bh = bfrag(cur, m2, dt);
+            f16x8 bl;
+            if constexpr (!FP8) bl = bfrag(cur + PLANE, m2, dt);
+            t = mma16(rc[m2], bh, t);
+            after(k++);
+            if constexpr (!FP8) {
+              g[dt] = mma16(ra[m2], bl, g[dt]);
+              after(k++);
+              t = mma16(rm[m2], bl, t);
+              after(k++);
+            }
+            g[dt] = mma16(ra[m2], bh, g[dt]);
+            after(k++);
+            t = mma16(rm[m2], bh, t);
+            after(k++);
+          }
+        };
+        auto fold = [&](int dt, const f32x16& t, int v0, int v1) {
+#pragma unroll
+          for (int v = v0; v < v1; ++v) g[dt][v] = fmaf(t[v], 1.0f / kRFine, g[dt][v]);
+        };
+        if constexpr (split_occ(DP, MODE) > 1) {
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) {
-            const f16x8 bh = bfrag(cur, m2, dt);
-            if constexpr (!FP8) g[dt] = mma16(rh[m2], bfrag(cur + PLANE, m2, dt), g[dt]);
-            g[dt] = mma16(rl[m2], bh, g[dt]);
-            g[dt] = mma16(rh[m2], bh, g[dt]);
+            f32x16 t;
+            products(dt, t, [](int) {});
+            fold(dt, t, 0, 16);
           }
+        } else {
+          // one wave per SIMD: a block's fine sums are added between the
+          // products of the next one
+          f32x16 t[2];
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt)
+            products(dt, t[dt & 1], [&](int k) {
+              if (dt > 0) fold(dt - 1, t[(dt - 1) & 1], 16 * k / NP, 16 * (k + 1) / NP);
+              __builtin_amdgcn_sched_barrier(0);
+            });
+          fold(DT - 1, t[(DT - 1) & 1], 0, 16);
+        }
       }
       if constexpr (!FP8) {
         // A of tile i + 2 and B of tile i + 1 must be there for the next
