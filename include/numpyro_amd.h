@@ -176,10 +176,10 @@ int nax_model_hier(nax_sampler* h, const float* d_x, const float* d_y, const int
  * n*d <= 2^20, d <= 64; otherwise, for d <= 256, row tiles on the fp32 matrix
  * cores below 32 chains, the VALU tile kernel or the matrix-core kernel,
  * whichever the autotuner times faster, up to 128 and the matrix-core kernel
- * above; the VALU tile kernel for 257 <= d <= 320), 1 = VALU
- * tile kernel, 2 = matrix cores (X Z^T in fp32; X^T R by two fp16 terms of X
- * and three of R where rows and column ranges allow, else fp32), 3 = one
- * wavefront per chain.  bf16 storage
+ * above; the VALU tile kernel for 257 <= d <= 320; the matrix-core kernel takes
+ * X Z^T in fp32 and X^T R by two fp16 terms of X and three of R where rows and
+ * column ranges allow, else in fp32 too), 1 = VALU tile kernel, 2 = matrix
+ * cores, both products in fp32, 3 = one wavefront per chain.  bf16 storage
  * always uses the matrix cores: 0 (auto) or 4 keep one bf16 copy of X and
  * read it transposed for X^T R with bf16 residuals; 2 keeps a second, fp16
  * copy for X^T R with fp16 residuals (twice the X bytes per evaluation, a

@@ -471,7 +471,8 @@ Potential* make_logistic_rows(const float* x, const float* y, int64_t n, int d,
 int64_t logistic_split_min_rows();
 Potential* make_logistic_split(const float* x, const uint8_t* codes, const float* scales,
                                const float* y, int64_t n, int d, double prior_scale,
-                               int num_chains, hipStream_t s, std::string* err);
+                               int num_chains, bool fp32_products, hipStream_t s,
+                               std::string* err);
 
 // fuse_variant: 0 = auto (fp32: row tiles below 32 chains, else matrix cores), 1 = VALU tile
 // kernel, 2 = matrix cores, 3 = a group of wavefronts per chain.  bf16 always runs on
@@ -513,7 +514,9 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
   const bool mfma = fp8 ? fuse_variant == 0 && d <= 256 && n >= logistic_split_min_rows()
                         : fuse_variant == 2 || (fuse_variant == 0 && num_chains >= 32 && d <= 256);
   auto matrix_form = [&](const uint8_t* codes, const float* scales) -> Potential* {
-    return make_logistic_split(x, codes, scales, y, n, d, prior_scale, num_chains, s, err);
+    // a caller that names the fp32 matrix kernel gets both products in fp32
+    return make_logistic_split(x, codes, scales, y, n, d, prior_scale, num_chains,
+                               fuse_variant == 2, s, err);
   };
   if (mfma && !fp8 && !(fuse_variant == 0 && num_chains <= 128 && d <= 320))
     return matrix_form(nullptr, nullptr);

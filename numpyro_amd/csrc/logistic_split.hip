@@ -713,7 +713,7 @@ struct LogisticSplit : Potential {
 
   // X fp32 row-major, or its codes and column scales (fp8).
   hipError_t setup(const float* x, const uint8_t* codes, const float* scales, const float* y,
-                   int num_chains, hipStream_t s) {
+                   int num_chains, bool fp32_products, hipStream_t s) {
     ntile = (n + 31) / 32;
     dp = (d + 31) / 32 * 32;
     int dev = 0;
@@ -727,7 +727,7 @@ struct LogisticSplit : Potential {
       e = hipMemcpyAsync(cscale, scales, sizeof(float) * d, hipMemcpyDeviceToDevice, s);
     } else {
       mode = kSplitF32;
-      bool ok = n >= kSplitMin && n <= kSplitRows * row_splits(num_chains);
+      bool ok = !fp32_products && n >= kSplitMin && n <= kSplitRows * row_splits(num_chains);
       if (ok) e = column_scales(x, s, &ok);
       if (!ok) mode = kPlainF32;
     }
@@ -813,10 +813,12 @@ struct LogisticSplit : Potential {
 int64_t logistic_split_min_rows() { return kSplitMin; }
 
 // fp32 X, or (codes given) its e4m3 codes [n][d] and column scales [d], which
-// are copied; d <= 256, n rows for num_chains chains.
+// are copied; d <= 256, n rows for num_chains chains.  fp32_products: X^T R on the
+// fp32 MFMA whatever the design.
 Potential* make_logistic_split(const float* x, const uint8_t* codes, const float* scales,
                                const float* y, int64_t n, int d, double prior_scale,
-                               int num_chains, hipStream_t s, std::string* err) {
+                               int num_chains, bool fp32_products, hipStream_t s,
+                               std::string* err) {
   if (d > 256) {
     *err = "the MFMA logistic kernels support dim <= 256";
     return nullptr;
@@ -825,7 +827,7 @@ Potential* make_logistic_split(const float* x, const uint8_t* codes, const float
   p->n = n;
   p->d = d;
   p->prior_scale = prior_scale;
-  const hipError_t e = p->setup(x, codes, scales, y, num_chains, s);
+  const hipError_t e = p->setup(x, codes, scales, y, num_chains, fp32_products, s);
   if (e != hipSuccess) {
     *err = std::string("logistic matrix-core setup: ") + hipGetErrorString(e);
     delete p;

@@ -1,4 +1,6 @@
-"""Small residuals in the matrix-core kernel's X^T R (logit_split_kernel): rare
+"""Precision of the matrix-core kernel's forms (logit_split_kernel).
+
+Small residuals in the matrix-core kernel's X^T R (logit_split_kernel): rare
 events on one-hot and binary columns, where thousands of rows share one residual
 far below 1 and an error of it has the same sign in all of them.
 
@@ -8,13 +10,18 @@ of sum |x z| =: M; the exponential's argument a = |l| log2 e carries 1.5 roundin
 2^-24 a, scaled by ln 2, and exp2, 1 + e, reciprocal and product together 6 of 2^-24;
 the sums over a row split take 5 roundings per 32 rows (two products of R's grid
 terms with each half tile, and the tile's fine terms), each at most 2^-24 of what
-the split holds.  A split has at most 512 of the 131,072 rows."""
+the split holds.  A split has at most 512 of the 131,072 rows.
+
+Products in fp32: at z = 0 a residual is +-1/2, and a column with one number x that
+is not zero has the gradient +-x/2 exactly; two fp16 terms of x miss its last bit
+now and then."""
 import math
 
 import pytest
 import torch
 
 from numpyro_amd import _lib
+from test_gpu_logistic_split import _check, _data
 
 pytestmark = pytest.mark.gpu
 
@@ -62,3 +69,28 @@ def test_rare_events_keep_their_bits(D, rate, x_dtype, C):
     eps = (2 * M + 1.5 * math.log(2) * 1.4427 * M + 6 + steps) * 2.0 ** -24
     bound = eps * (r.abs().T.contiguous() @ x.abs()) + 2.0 ** -23 * z64.abs() + 1e-9
     assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
+
+
+def _single_entries(C):
+    """64 columns of one number each, 24 bits long, in rows of their own."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    X = torch.zeros((65536, 64), device="cuda")
+    rows = torch.randperm(65536, generator=g, device="cuda")[:64]
+    X[rows, torch.arange(64, device="cuda")] = 1 + torch.rand(64, generator=g, device="cuda")
+    y = (torch.rand(65536, generator=g, device="cuda") < 0.5).float()
+    want = (X[rows].amax(1) * (0.5 - y[rows])).double()
+    return X, y, torch.zeros((C, 64), device="cuda"), want
+
+
+def test_named_matrix_kernel_multiplies_in_fp32():
+    X, y, z, want = _single_entries(40)
+    assert torch.equal(_grad(X, y, z, "fp32", "mfma"), want.expand(40, 64))
+
+
+@pytest.mark.parametrize("N, D, C", [(65536, 1, 129), (65537, 31, 130), (65567, 33, 130),
+                                     (65568, 64, 300), (100003, 97, 129), (65537, 128, 130),
+                                     (65537, 129, 130), (65537, 193, 129), (65569, 225, 130),
+                                     (65537, 256, 300)])
+def test_automatic_choice_at_the_edges_of_its_tiles(N, D, C):
+    """Above 128 chains the automatic choice is the form in fp16 terms."""
+    _check(*_data(N, D, C, N + D), kernel="auto")
