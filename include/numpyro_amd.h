@@ -177,16 +177,16 @@ int nax_model_hier(nax_sampler* h, const float* d_x, const float* d_y, const int
  * cores below 32 chains, the VALU tile kernel or the matrix-core kernel,
  * whichever the autotuner times faster, up to 128 and the matrix-core kernel
  * above; the VALU tile kernel for 257 <= d <= 320; the matrix-core kernel takes
- * X Z^T in fp32 and X^T R by two fp16 terms of X and three of R where rows and
- * column ranges allow, else in fp32 too), 1 = VALU tile kernel, 2 = matrix
+ * X Z^T in fp32 and X^T R by two fp16 terms of X and three of R where rows, column
+ * ranges and labels allow, else in fp32 too), 1 = VALU tile kernel, 2 = matrix
  * cores, both products in fp32, 3 = one wavefront per chain.  bf16 storage
  * always uses the matrix cores: 0 (auto) or 4 keep one bf16 copy of X and
  * read it transposed for X^T R with bf16 residuals; 2 keeps a second, fp16
  * copy for X^T R with fp16 residuals (twice the X bytes per evaluation, a
  * gradient rounding of 2^-11 instead of 2^-8 per term, and max|X| < 60000).
  * fp8 storage (NAX_X_FP8; the library quantises d_x as nax_fp8_quantize
- * does and keeps the codes): 0 (auto: the matrix cores for d <= 256 and
- * n >= 65536, else the VALU tile kernel with autotuned row splits) or 1 (VALU
+ * does and keeps the codes): 0 (auto: the matrix cores for d <= 256,
+ * n >= 65536 and labels in [0, 1], else the VALU tile kernel with autotuned row splits) or 1 (VALU
  * tile kernel).  Other kernel values with bf16 or fp8 storage,
  * and 4 with fp32 storage, are refused (NAX_EINVAL). */
 int nax_model_logistic_ex(nax_sampler* h, const float* d_x, const float* d_y, int64_t n,

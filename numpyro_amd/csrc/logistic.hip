@@ -469,6 +469,7 @@ Potential* make_logistic_rows(const float* x, const float* y, int64_t n, int d,
                               double prior_scale);
 
 int64_t logistic_split_min_rows();
+hipError_t logistic_split_labels(const float* y, int64_t n, hipStream_t s, bool* ok);
 Potential* make_logistic_split(const float* x, const uint8_t* codes, const float* scales,
                                const float* y, int64_t n, int d, double prior_scale,
                                int num_chains, bool fp32_products, hipStream_t s,
@@ -510,9 +511,16 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
   // of chains (the tile kernel takes 8 chains at a time through a table lookup
   // per element; a call at 500,000 x 250: 250 chains 15.0 ms against 1.0, 32 chains
   // 2.24 against 0.68, 1 chain 0.94 against 0.62; 70,000 x 30, 2 chains 0.35 against
-  // 0.22)
-  const bool mfma = fp8 ? fuse_variant == 0 && d <= 256 && n >= logistic_split_min_rows()
-                        : fuse_variant == 2 || (fuse_variant == 0 && num_chains >= 32 && d <= 256);
+  // 0.22), for labels in [0, 1]
+  bool mfma = fp8 ? fuse_variant == 0 && d <= 256 && n >= logistic_split_min_rows()
+                  : fuse_variant == 2 || (fuse_variant == 0 && num_chains >= 32 && d <= 256);
+  if (fp8 && mfma) {
+    const hipError_t e = logistic_split_labels(y, n, s, &mfma);
+    if (e != hipSuccess) {
+      *err = std::string("logistic labels: ") + hipGetErrorString(e);
+      return nullptr;
+    }
+  }
   auto matrix_form = [&](const uint8_t* codes, const float* scales) -> Potential* {
     // a caller that names the fp32 matrix kernel gets both products in fp32
     return make_logistic_split(x, codes, scales, y, n, d, prior_scale, num_chains,

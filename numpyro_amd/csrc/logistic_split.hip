@@ -44,7 +44,8 @@
 // two (exact): column d of X such that max |X'_d| lies in [2^14, 2^15), R by
 // 2^14.  A term of 2^-39 of its column's largest is then still represented.
 // The split takes a design whose columns are finite with max |X_d| <= 2^12
-// rms(X_d), so that this is below fp32's own rounding of a typical element.
+// rms(X_d), so that this is below fp32's own rounding of a typical element, and
+// labels in [0, 1] (|r| <= 1; fp16 ends at |R'| = 2^16).
 // Its number of rows is bounded too: on more than kSplitRows rows per partial
 // sum the fp32 accumulators' own rounding reaches 1e-5 of the gradient
 // (N = 2,000,000, 1024 chains: 9e-6 to 2e-5), and results would differ by it
@@ -158,6 +159,17 @@ split_col_scale(const unsigned* __restrict__ pmax, const double* __restrict__ ps
   if (ok) frexp(sqrt(s / (double)N) / sc, &e);  // rms of the scaled column in [2^(e-1), 2^e)
   cgrid[d] = ldexpf(1.0f, e - 11);
   if (!ok) atomicAdd(bad, 1);
+}
+
+// Adds the labels outside [0, 1] to *bad: a residual of 4 or more is past fp16
+// after R's scale.
+__global__ void __launch_bounds__(256)
+split_label_range(const float* __restrict__ y, int64_t N, int* __restrict__ bad) {
+  int k = 0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N;
+       i += (int64_t)gridDim.x * blockDim.x)
+    k += !(y[i] >= 0.0f && y[i] <= 1.0f);
+  if (k) atomicAdd(bad, k);
 }
 
 // GEMM1's fp32 order: out[T][q][lane][j] = X[32 T + lane % 32][8 q + 2 j + lane / 32],
@@ -687,8 +699,8 @@ struct LogisticSplit : Potential {
     return (int)std::min<int64_t>(RB, (ntile + 7) / 8 * 8);
   }
 
-  // The split of GEMM2 takes the design (fp32): the range rule of the header.
-  hipError_t column_scales(const float* x, hipStream_t s, bool* ok) {
+  // The split of GEMM2 takes the design (fp32): the range rules of the header.
+  hipError_t column_scales(const float* x, const float* y, hipStream_t s, bool* ok) {
     char* tmp = nullptr;  // [blocks][d] doubles, then bits, then the count
     const size_t cells = (size_t)kStatBlocks * d;
     hipError_t e = hipMallocAsync((void**)&tmp, cells * 12 + sizeof(int), s);
@@ -702,6 +714,7 @@ struct LogisticSplit : Potential {
       hipLaunchKernelGGL(split_col_stats, dim3(kStatBlocks), dim3(256), 0, s, x, n, d, pmax, psq);
       hipLaunchKernelGGL(split_col_scale, dim3(1), dim3(256), 0, s, pmax, psq, kStatBlocks, n, d,
                          cscale, cscale + d, bad);
+      hipLaunchKernelGGL(split_label_range, dim3(256), dim3(256), 0, s, y, n, bad);
       e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s);
@@ -728,7 +741,7 @@ struct LogisticSplit : Potential {
     } else {
       mode = kSplitF32;
       bool ok = !fp32_products && n >= kSplitMin && n <= kSplitRows * row_splits(num_chains);
-      if (ok) e = column_scales(x, s, &ok);
+      if (ok) e = column_scales(x, y, s, &ok);
       if (!ok) mode = kPlainF32;
     }
     if (e != hipSuccess) return e;
@@ -811,6 +824,24 @@ struct LogisticSplit : Potential {
 };
 
 int64_t logistic_split_min_rows() { return kSplitMin; }
+
+// Whether every label is in [0, 1], as the forms in fp16 terms need it.
+hipError_t logistic_split_labels(const float* y, int64_t n, hipStream_t s, bool* ok) {
+  int* bad = nullptr;
+  int hbad = 0;
+  hipError_t e = hipMallocAsync((void**)&bad, sizeof(int), s);
+  if (e != hipSuccess) return e;
+  e = hipMemsetAsync(bad, 0, sizeof(int), s);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(split_label_range, dim3(256), dim3(256), 0, s, y, n, bad);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  (void)hipFreeAsync(bad, s);
+  *ok = hbad == 0;
+  return e;
+}
 
 // fp32 X, or (codes given) its e4m3 codes [n][d] and column scales [d], which
 // are copied; d <= 256, n rows for num_chains chains.  fp32_products: X^T R on the

@@ -21,7 +21,7 @@ import pytest
 import torch
 
 from numpyro_amd import _lib
-from test_gpu_logistic_split import _check, _data
+from test_gpu_logistic_split import _check, _data, _stored
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +94,21 @@ def test_named_matrix_kernel_multiplies_in_fp32():
 def test_automatic_choice_at_the_edges_of_its_tiles(N, D, C):
     """Above 128 chains the automatic choice is the form in fp16 terms."""
     _check(*_data(N, D, C, N + D), kernel="auto")
+
+
+@pytest.mark.filterwarnings("ignore:Out-of-support values")
+@pytest.mark.parametrize("label", [4.5, -7.0, 1e6])
+@pytest.mark.parametrize("x_dtype, C", [("fp32", 130), ("fp8", 33)])
+def test_labels_outside_the_unit_interval(x_dtype, C, label):
+    """A residual past fp16's range: the design takes the kernels in fp32.  Bound of
+    a gradient entry: test_gpu_logistic_split's for a chain of fp32 multiply-adds."""
+    X, y, z = _data(65600, 24, C, 6)
+    y[1234] = label
+    got = _grad(X, y, z, x_dtype, "auto")
+    x, z64 = _stored(X, x_dtype), z.double()
+    r = torch.sigmoid(x @ z64.T) - y.double()[:, None]
+    want = r.T.contiguous() @ x + z64
+    dr = 2.0 ** -21 + 0.25 * 25 * 2.0 ** -24 * (x.abs() @ z64.abs().T)
+    bound = dr.T.contiguous() @ x.abs() \
+        + (2.0 ** -21 + 65600 / 8 * 2.0 ** -24) * (r.abs().T.contiguous() @ x.abs()) + 1e-6
+    assert ((got - want).abs() <= bound).all()
