@@ -305,13 +305,15 @@ __device__ __forceinline__ float softplusf_(float x) {
 }
 
 // log1p(e) for e in [0, 1], as 2 atanh(s) with s = e / (2 + e) <= 1/3: the
-// odd series up to s^17 (next term 2e-9), every step rounded to nearest.
-// A quarter of log1pf's instructions.
+// odd series up to s^17 (next term 2e-9).  What the rounding of s leaves out (lo) is
+// added to the series, so that the result is rounded about once, as log1pf's is;
+// half its instructions.
 __device__ __forceinline__ float log1p_unit(float e) {
+#pragma clang fp contract(off)
   const float den = 2.0f + e;
   const float inv = __builtin_amdgcn_rcpf(den);
-  const float s0 = e * inv;
-  const float s = fmaf(fmaf(-s0, den, e), inv, s0);
+  const float s = e * inv;
+  const float lo = fmaf(-s, e - (den - 2.0f), fmaf(-s, den, e)) * inv;
   const float t = s * s;
   float p = 1.0f / 17.0f;
   p = fmaf(p, t, 1.0f / 15.0f);
@@ -322,14 +324,25 @@ __device__ __forceinline__ float log1p_unit(float e) {
   p = fmaf(p, t, 1.0f / 5.0f);
   p = fmaf(p, t, 1.0f / 3.0f);
   const float s2 = s + s;
-  return fmaf(s2 * t, p, s2);
+  return s2 + fmaf(s2 * t, p, lo + lo);
 }
 
-// The terms with log1p (exact for small e, where log2(1 + e) has lost e's low
-// bits, as the VALU tile kernel has them), r as above.
+// r = sigmoid(l) - y and u = softplus(l) - y l with log1p (exact for small e, where
+// log2(1 + e) has lost e's low bits) and the quotient's remainder added to q - y:
+// no further from float64 than sigmoidf_ and softplusf_ with their division and
+// log1pf.  Root mean square errors over 2^20 logits, (r, u) of this / of those:
+// l in (-6, -2), y = 0 (3.2e-9, 3.4e-9) / (3.4e-9, 3.5e-9); l in (0, 2), y = 0
+// (1.9e-8, 3.8e-8) / (2.7e-8, 3.8e-8); with the quotient as it comes and no lo in
+// log1p_unit (3.6e-9, 3.9e-9) and (2.9e-8, 4.1e-8).
 __device__ __forceinline__ void logit_terms_log1p(float l, float y, float& r, float& u) {
+#pragma clang fp contract(off)
   const float e = __expf(-fabsf(l));
-  r = fmaf(l >= 0.0f ? 1.0f : e, __builtin_amdgcn_rcpf(1.0f + e), -y);
+  const float d = 1.0f + e;
+  const float inv = __builtin_amdgcn_rcpf(d);
+  const float num = l >= 0.0f ? 1.0f : e;
+  const float q = num * inv;
+  const float rem = fmaf(-q, e - (d - 1.0f), fmaf(-q, d, num));
+  r = fmaf(rem, inv, q - y);
   u = fmaf(-y, l, fmaxf(l, 0.0f) + log1p_unit(e));
 }
 

@@ -112,3 +112,33 @@ def test_labels_outside_the_unit_interval(x_dtype, C, label):
     bound = dr.T.contiguous() @ x.abs() \
         + (2.0 ** -21 + 65600 / 8 * 2.0 ** -24) * (r.abs().T.contiguous() @ x.abs()) + 1e-6
     assert ((got - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("label", [0.0, 1.0])
+@pytest.mark.parametrize("lo, hi", [(-12.0, -6.0), (-6.0, -2.0), (-2.0, 0.0), (0.0, 2.0),
+                                    (2.0, 6.0), (6.0, 12.0)])
+def test_fp8_residuals_are_as_exact_as_the_tile_kernels(lo, hi, label):
+    """Each of 64 columns has a 1 in one row, so that its gradient is that row's
+    residual (the prior's part is 1e-12 of z).  250 x 64 residuals: their root mean
+    square error from float64 varies by about 1 / sqrt(2 16000) = 0.6 % between samples
+    of the same accuracy, hence 1.02."""
+    from numpyro_amd.infer.hmc import Engine
+    from numpyro_amd.models import LogisticRegression
+    g = torch.Generator(device="cuda").manual_seed(8)
+    X = torch.zeros((65536, 64), device="cuda")
+    rows = torch.randperm(65536, generator=g, device="cuda")[:64]
+    X[rows, torch.arange(64, device="cuda")] = 1.0
+    y = torch.full((65536,), label, device="cuda")
+    z = lo + (hi - lo) * torch.rand((250, 64), generator=g, device="cuda")
+    want = torch.sigmoid(z.double()) if label == 0.0 else -torch.sigmoid(-z.double())
+    err = {}
+    for kernel in ("auto", "tile"):
+        model = LogisticRegression(X, y, prior_scale=1e6, x_dtype="fp8", kernel=kernel)
+        eng = Engine(model, 250, "NUTS", 0)
+        pe = torch.empty(250, dtype=torch.float64, device="cuda")
+        got = torch.empty((250, 64), device="cuda")
+        torch.cuda.synchronize()
+        _lib.check(_lib.load().nax_potential_grad(eng.h, _lib.ptr(z), 64, 250, _lib.ptr(pe),
+                                                  _lib.ptr(got)), "potential_grad")
+        err[kernel] = float((got.double() - 1e-12 * z.double() - want).square().mean().sqrt())
+    assert err["auto"] <= 1.02 * err["tile"], err
