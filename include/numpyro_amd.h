@@ -186,9 +186,9 @@ int nax_model_hier(nax_sampler* h, const float* d_x, const float* d_y, const int
  * gradient rounding of 2^-11 instead of 2^-8 per term, and max|X| < 60000).
  * fp8 storage (NAX_X_FP8; the library quantises d_x as nax_fp8_quantize
  * does and keeps the codes): 0 (auto: the matrix cores for d <= 256,
- * n >= 65536 and labels in [0, 1], else the VALU tile kernel with autotuned row splits) or 1 (VALU
- * tile kernel).  Other kernel values with bf16 or fp8 storage,
- * and 4 with fp32 storage, are refused (NAX_EINVAL). */
+ * n >= 65536 and labels in [0, 1], else the VALU tile kernel with autotuned row
+ * splits) or 1 (VALU tile kernel).  Other kernel values with bf16 or fp8
+ * storage, and 4 with fp32 storage, are refused (NAX_EINVAL). */
 int nax_model_logistic_ex(nax_sampler* h, const float* d_x, const float* d_y, int64_t n,
                           int32_t d, double prior_scale, int32_t x_dtype, int32_t kernel);
 
@@ -324,10 +324,10 @@ int nax_potential_grad(nax_sampler* h, const float* d_z, int32_t ld, int32_t cou
 
 /* The same enqueued on the caller's stream (a hipStream_t; NULL = the null
  * stream) without waiting for it: pe and grad are written in stream order.
- * Calls on several streams or threads are ordered behind one another (they
- * share the model's workspaces), and so are the sampler's own calls behind
- * them; none may run beside nax_run on the same sampler.  A subsampled model's
- * indices must not be under update (nax_ecs_gibbs) when it is called. */
+ * Calls on several streams or threads are ordered behind one another and behind
+ * nax_ecs_gibbs (they share the model's workspaces and indices), and so are the
+ * sampler's own calls behind them; none may run beside nax_run on the same
+ * sampler. */
 int nax_potential_grad_on(nax_sampler* h, const float* d_z, int32_t ld, int32_t count,
                           double* d_pe, float* d_grad, void* stream);
 

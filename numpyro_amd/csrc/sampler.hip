@@ -268,12 +268,15 @@ struct nax_sampler {
   double timing_ms = 0.0;
   int64_t timing_n = 0;
   std::vector<hipEvent_t> ev;
-  // nax_potential_grad_on: recorded behind the last evaluation on a caller's
-  // stream; whatever uses the model's workspaces next on another stream waits
-  // for it
+  // Recorded behind the last work that left the model's workspaces in use when its
+  // call returned (nax_potential_grad_on, nax_ecs_gibbs); whatever uses them next
+  // waits for it.  The wait is never skipped: a stream's handle does not name the
+  // stream (hipStreamPerThread is another one in every thread, and a destroyed
+  // stream's handle can come back), and behind itself a stream waits for nothing.
+  // on_mu is held while work is enqueued, and by calls that wait for their own work
+  // until they have.
   std::mutex on_mu;
   hipEvent_t on_done = nullptr;
-  hipStream_t on_stream = nullptr;
   bool on_pending = false;
 };
 
@@ -290,12 +293,18 @@ static const int kBatch = 16;
 
 extern "C" const char* nax_last_error(void) { return g_err.c_str(); }
 
-// Orders the sampler's own stream behind evaluations on callers' streams.
-static hipError_t wait_callers(nax_sampler* h) {
-  std::lock_guard<std::mutex> lk(h->on_mu);
-  if (!h->on_pending) return hipSuccess;
-  h->on_pending = false;
-  return hipStreamWaitEvent(h->stream, h->on_done, 0);
+// Orders stream s behind the last user of the workspaces (on_mu held).
+static hipError_t wait_last(nax_sampler* h, hipStream_t s) {
+  return h->on_pending ? hipStreamWaitEvent(s, h->on_done, 0) : hipSuccess;
+}
+// Stream s is the last user (on_mu held).
+static hipError_t record_last(nax_sampler* h, hipStream_t s) {
+  if (!h->on_done) {
+    const hipError_t e = hipEventCreateWithFlags(&h->on_done, hipEventDisableTiming);
+    if (e != hipSuccess) return e;
+  }
+  h->on_pending = true;
+  return hipEventRecord(h->on_done, s);
 }
 
 static std::vector<int> schedule_ends(int num_steps) {
@@ -515,9 +524,11 @@ extern "C" int nax_ecs_gibbs(nax_sampler* h, float* accept_prob) {
   if (!h->initialized) { set_error("nax_ecs_gibbs before nax_init"); return NAX_ESTATE; }
   if (!h->pot) { set_error("nax_ecs_gibbs: no subsampled model set"); return NAX_ESTATE; }
   const EngineCfg& e = h->cfg;
-  NAX_HIP(wait_callers(h));
+  std::lock_guard<std::mutex> lk(h->on_mu);
+  NAX_HIP(wait_last(h, h->stream));
   hipError_t r = h->pot->ecs_gibbs(h->stream, h->st, h->vec + (size_t)V_Z * e.Dp,
                                    h->vec + (size_t)V_G * e.Dp, e.nvec * e.Dp, accept_prob);
+  NAX_HIP(record_last(h, h->stream));
   if (r == hipErrorNotSupported) {
     set_error("nax_ecs_gibbs: the model has no subsample plate (use nax_model_logistic_ecs)");
     return NAX_ESTATE;
@@ -654,7 +665,8 @@ extern "C" int nax_init(nax_sampler* h, const float* z0, const uint32_t* keys,
   if (!h || !z0 || !keys) { set_error("nax_init: null argument"); return NAX_EINVAL; }
   if (!h->pot && !h->external) { set_error("nax_init: no model set"); return NAX_ESTATE; }
   const EngineCfg& e = h->cfg;
-  NAX_HIP(wait_callers(h));
+  std::lock_guard<std::mutex> lk(h->on_mu);
+  NAX_HIP(wait_last(h, h->stream));
   uint32_t* dkeys = nullptr;
   NAX_HIP(hipMallocAsync((void**)&dkeys, sizeof(uint32_t) * 2 * e.C, h->stream));
   NAX_HIP(hipMemcpyAsync(dkeys, keys, sizeof(uint32_t) * 2 * e.C, hipMemcpyHostToDevice, h->stream));
@@ -696,7 +708,10 @@ extern "C" int nax_run(nax_sampler* h, int64_t target, const nax_collect* c, int
   if (!h->initialized) { set_error("nax_run before nax_init"); return NAX_ESTATE; }
   if (h->external || !h->pot) { set_error("nax_run needs a built-in model; use nax_advance"); return NAX_ESTATE; }
   Collect col = to_collect(c);
-  NAX_HIP(wait_callers(h));
+  {
+    std::lock_guard<std::mutex> lk(h->on_mu);
+    NAX_HIP(wait_last(h, h->stream));
+  }
   NAX_HIP(hipMemsetAsync(h->gevals, 0, sizeof(int64_t), h->stream));
   if (h->pot->persistent()) {
     // Whole loop on the device, in chunks of iterations with progress
@@ -1033,7 +1048,8 @@ extern "C" int nax_potential_grad(nax_sampler* h, const float* z, int32_t ld, in
   if (!h || !z || !pe || !g) { set_error("null argument"); return NAX_EINVAL; }
   if (!h->pot) { set_error("no built-in model set"); return NAX_ESTATE; }
   if (count <= 0 || ld < h->cfg.D) { set_error("bad count / ld"); return NAX_EINVAL; }
-  NAX_HIP(wait_callers(h));
+  std::lock_guard<std::mutex> lk(h->on_mu);
+  NAX_HIP(wait_last(h, h->stream));
   NAX_HIP(h->pot->eval(h->stream, z, ld, count, pe, g, ld));
   NAX_HIP(hipStreamSynchronize(h->stream));
   return NAX_OK;
@@ -1050,13 +1066,10 @@ extern "C" int nax_potential_grad_on(nax_sampler* h, const float* z, int32_t ld,
   if (count <= 0 || ld < h->cfg.D) { set_error("bad count / ld"); return NAX_EINVAL; }
   hipStream_t s = static_cast<hipStream_t>(stream);
   std::lock_guard<std::mutex> lk(h->on_mu);
-  if (!h->on_done)
-    NAX_HIP(hipEventCreateWithFlags(&h->on_done, hipEventDisableTiming));
-  if (h->on_pending && h->on_stream != s) NAX_HIP(hipStreamWaitEvent(s, h->on_done, 0));
-  NAX_HIP(h->pot->eval(s, z, ld, count, pe, g, ld));
-  NAX_HIP(hipEventRecord(h->on_done, s));
-  h->on_stream = s;
-  h->on_pending = true;
+  NAX_HIP(wait_last(h, s));
+  const hipError_t r = h->pot->eval(s, z, ld, count, pe, g, ld);
+  NAX_HIP(record_last(h, s));  // also behind the part that a failed call enqueued
+  NAX_HIP(r);
   return NAX_OK;
 }
 
@@ -1065,7 +1078,8 @@ extern "C" int nax_leapfrog(nax_sampler* h, float* z, float* r, float* g, double
   if (!h || !z || !r || !g || !pe || !imm) { set_error("null argument"); return NAX_EINVAL; }
   if (!h->pot) { set_error("no built-in model set"); return NAX_ESTATE; }
   const EngineCfg& e = h->cfg;
-  NAX_HIP(wait_callers(h));
+  std::lock_guard<std::mutex> lk(h->on_mu);
+  NAX_HIP(wait_last(h, h->stream));
   dim3 grid((e.D + 127) / 128, e.C);
   for (int s = 0; s < L; ++s) {
     hipLaunchKernelGGL(lf_half_kernel, grid, dim3(128), 0, h->stream, e.C, e.D, e.D, z, r, g,
