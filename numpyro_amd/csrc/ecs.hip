@@ -567,17 +567,16 @@ struct EcsLogistic : Potential {
   double* pe_new = nullptr;
   float* g_new = nullptr;
   double* buf = nullptr;  // bref, per-row scalars, G, H
-  // H delta of each chain [hd_chains][d], degree 2: one for evaluations, one for the
-  // Gibbs update, which a caller's evaluation on another stream may overlap
-  double* hd_of[2] = {nullptr, nullptr};
-  int hd_chains[2] = {0, 0};
+  // H delta of each chain [hd_chains][d], degree 2; evaluations and Gibbs updates
+  // of a sampler are ordered behind one another
+  double* hd = nullptr;
+  int hd_chains = 0;
   ~EcsLogistic() override {
     (void)hipFree(prop);
     (void)hipFree(pe_new);
     (void)hipFree(g_new);
     (void)hipFree(buf);
-    (void)hipFree(hd_of[0]);
-    (void)hipFree(hd_of[1]);
+    (void)hipFree(hd);
   }
   int dim() const override { return a.d; }
   const char* name() const override { return "ecs_eval_kernel"; }
@@ -589,19 +588,18 @@ struct EcsLogistic : Potential {
   }
   double alg_flops(int C_) const override { return 4.0 * C_ * a.m * a.d; }
   hipError_t launch(hipStream_t s, const int* ix, const float* z, int ldz, int grid, const int* act,
-                    const int* nact, double* pe, float* g, int ldg, bool gibbs = false) {
-    const bool mark = !gibbs;
+                    const int* nact, double* pe, float* g, int ldg, bool mark = true) {
     if (a.proxy == 2) {
-      if (grid > hd_chains[gibbs]) {
-        (void)hipFree(hd_of[gibbs]);
-        hd_of[gibbs] = nullptr;
-        hd_chains[gibbs] = 0;
-        const hipError_t e = hipMalloc(&hd_of[gibbs], sizeof(double) * (size_t)grid * a.d);
+      if (grid > hd_chains) {
+        (void)hipFree(hd);
+        hd = nullptr;
+        hd_chains = 0;
+        const hipError_t e = hipMalloc(&hd, sizeof(double) * (size_t)grid * a.d);
         if (e != hipSuccess) return e;
-        hd_chains[gibbs] = grid;
+        hd_chains = grid;
       }
       hipLaunchKernelGGL(ecs_proxy_kernel, dim3((grid + kProxyChains - 1) / kProxyChains),
-                         dim3(kEcsThreads * kProxyParts), 0, s, a, z, ldz, grid, act, nact, hd_of[gibbs]);
+                         dim3(kEcsThreads * kProxyParts), 0, s, a, z, ldz, grid, act, nact, hd);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
     }
@@ -611,7 +609,7 @@ struct EcsLogistic : Potential {
     // with the proxy's kernel, 257 on four 78.
 #define NAX_ECS_NW(NCHV, RV, NWV)                                                             \
   hipLaunchKernelGGL(HIP_KERNEL_NAME(ecs_eval_kernel<NCHV, RV, NWV>), dim3(grid),                \
-                     dim3(NWV * NAX_WAVE), 0, s, a, ix, z, ldz, hd_of[gibbs], act, nact, pe, g, ldg)
+                     dim3(NWV * NAX_WAVE), 0, s, a, ix, z, ldz, hd, act, nact, pe, g, ldg)
 #define NAX_ECS(NCHV, RV)                            \
   do {                                               \
     if (grid <= 256) NAX_ECS_NW(NCHV, RV, 8);        \
@@ -647,7 +645,7 @@ struct EcsLogistic : Potential {
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     // U and dU at each chain's current position with the proposed indices
-    err = launch(s, prop, z, ldv, C, nullptr, nullptr, pe_new, g_new, Dp, true);
+    err = launch(s, prop, z, ldv, C, nullptr, nullptr, pe_new, g_new, Dp, false);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(ecs_accept_kernel, dim3(C), dim3(kEcsThreads), 0, s, C, a.m, a.d, part,
                        keys, pe_new, g_new, Dp, prop, idx, st, gst, ldv, accept);
@@ -686,11 +684,9 @@ Potential* make_ecs_logistic(const float* x, const float* y, int64_t n, int d, d
   if ((e = hipMalloc(&p->g_new, sizeof(float) * (size_t)num_chains * Dp))) return fail("hipMalloc", e);
   if (!proxy) return p;
   if (proxy == 2) {
-    for (int u = 0; u < 2; ++u) {
-      if ((e = hipMalloc(&p->hd_of[u], sizeof(double) * (size_t)num_chains * d)))
-        return fail("hipMalloc", e);
-      p->hd_chains[u] = num_chains;
-    }
+    if ((e = hipMalloc(&p->hd, sizeof(double) * (size_t)num_chains * d)))
+      return fail("hipMalloc", e);
+    p->hd_chains = num_chains;
   }
   // [rows: n records of 4 doubles][bref d][G d][H d*d]
   const size_t nbuf = 4 * (size_t)n + d + d + (size_t)d * d;
