@@ -567,10 +567,9 @@ struct EcsLogistic : Potential {
   double* pe_new = nullptr;
   float* g_new = nullptr;
   double* buf = nullptr;  // bref, per-row scalars, G, H
-  // H delta of each chain [hd_chains][d], degree 2; evaluations and Gibbs updates
-  // of a sampler are ordered behind one another
+  // H delta of each chain [C][d], degree 2; evaluations and Gibbs updates of a
+  // sampler are ordered behind one another
   double* hd = nullptr;
-  int hd_chains = 0;
   ~EcsLogistic() override {
     (void)hipFree(prop);
     (void)hipFree(pe_new);
@@ -589,15 +588,8 @@ struct EcsLogistic : Potential {
   double alg_flops(int C_) const override { return 4.0 * C_ * a.m * a.d; }
   hipError_t launch(hipStream_t s, const int* ix, const float* z, int ldz, int grid, const int* act,
                     const int* nact, double* pe, float* g, int ldg, bool mark = true) {
+    if (grid > C) return hipErrorInvalidValue;  // idx and hd have C rows
     if (a.proxy == 2) {
-      if (grid > hd_chains) {
-        (void)hipFree(hd);
-        hd = nullptr;
-        hd_chains = 0;
-        const hipError_t e = hipMalloc(&hd, sizeof(double) * (size_t)grid * a.d);
-        if (e != hipSuccess) return e;
-        hd_chains = grid;
-      }
       hipLaunchKernelGGL(ecs_proxy_kernel, dim3((grid + kProxyChains - 1) / kProxyChains),
                          dim3(kEcsThreads * kProxyParts), 0, s, a, z, ldz, grid, act, nact, hd);
       const hipError_t e = hipGetLastError();
@@ -683,11 +675,8 @@ Potential* make_ecs_logistic(const float* x, const float* y, int64_t n, int d, d
   if ((e = hipMalloc(&p->pe_new, sizeof(double) * num_chains))) return fail("hipMalloc", e);
   if ((e = hipMalloc(&p->g_new, sizeof(float) * (size_t)num_chains * Dp))) return fail("hipMalloc", e);
   if (!proxy) return p;
-  if (proxy == 2) {
-    if ((e = hipMalloc(&p->hd, sizeof(double) * (size_t)num_chains * d)))
-      return fail("hipMalloc", e);
-    p->hd_chains = num_chains;
-  }
+  if (proxy == 2 && (e = hipMalloc(&p->hd, sizeof(double) * (size_t)num_chains * d)))
+    return fail("hipMalloc", e);
   // [rows: n records of 4 doubles][bref d][G d][H d*d]
   const size_t nbuf = 4 * (size_t)n + d + d + (size_t)d * d;
   if ((e = hipMalloc(&p->buf, sizeof(double) * nbuf))) return fail("hipMalloc", e);

@@ -358,6 +358,9 @@ def _device_value_and_grad(model, z):
     C = int(z.shape[0])
     if hasattr(model, "bind"):
         model.bind(C)
+    idx = getattr(model, "idx", None)
+    if idx is not None and idx.shape[0] < C:
+        raise ValueError(f"z has {C} chains, the model the subsamples of {idx.shape[0]}")
     cache = model.__dict__.setdefault("_vg_engines", {})
     eng = cache.get(C)
     if eng is None:

@@ -1,6 +1,6 @@
 """Calls that share a model's workspaces, enqueued where a stream's handle does not
 tell the streams apart or where the last user is the sampler itself: each gives
-the bits that it gives alone."""
+the bits that it gives alone.  And the chains that such a call may ask for."""
 import threading
 
 import numpy as np
@@ -140,3 +140,24 @@ def test_evaluations_around_a_gibbs_update(degree):
     assert not torch.equal(idx, model.idx)
     for (u, g), (wu, wg) in zip(got, (before, after)):
         assert torch.equal(u, wu) and torch.equal(g, wg)
+
+
+@pytest.mark.parametrize("degree", [0, 2])
+def test_more_chains_than_subsamples_are_refused(degree):
+    from numpyro_amd.infer.hmc import Engine
+    from numpyro_amd.models import SubsampledLogisticRegression, potential_energy
+    X = np.random.default_rng(0).normal(size=(200, 3)).astype(np.float32)
+    model = SubsampledLogisticRegression(X, np.zeros(200, np.float32), 10, proxy_degree=degree,
+                                         reference=np.zeros(3) if degree else None)
+    model.idx = torch.zeros((4, 10), dtype=torch.int32, device="cuda")
+    model.keys = torch.zeros((4, 2), dtype=torch.int32, device="cuda")
+    eng = Engine(model, 4, "NUTS", 0)
+    z = torch.zeros((5, 3), device="cuda")
+    pe, g = torch.zeros(5, dtype=torch.float64, device="cuda"), torch.zeros((5, 3), device="cuda")
+    torch.cuda.synchronize()
+    for call, tail in ((eng.lib.nax_potential_grad, ()), (eng.lib.nax_potential_grad_on, (None,))):
+        args = (_lib.ptr(z), 3, 5, _lib.ptr(pe), _lib.ptr(g)) + tail
+        assert call(eng.h, *args) != 0
+    with pytest.raises(ValueError, match="subsamples of 4"):
+        potential_energy(model, z)
+    assert torch.isfinite(potential_energy(model, z[:4])).all()
