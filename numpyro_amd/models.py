@@ -363,12 +363,15 @@ def _device_value_and_grad(model, z):
         raise ValueError(f"z has {C} chains, the model the subsamples of {idx.shape[0]}")
     cache = model.__dict__.setdefault("_vg_engines", {})
     eng = cache.get(C)
-    if eng is None:
-        eng = cache[C] = Engine(model, C, "NUTS", 0)
     if torch.cuda.is_current_stream_capturing():
         # a graph would keep the addresses of the model's workspaces
         raise RuntimeError("potential_energy cannot be captured in a graph (see "
                            "nax_logistic_potential_grad_noalloc)")
+    if eng is None:
+        # the model's data may be on its way on another stream; the set-up runs on
+        # the sampler's own, and later calls are in stream order with this one
+        torch.cuda.synchronize()
+        eng = cache[C] = Engine(model, C, "NUTS", 0)
     D = model.dim
     zp = z.detach().to(device="cuda", dtype=torch.float32).contiguous()
     pe = torch.empty(C, dtype=torch.float64, device="cuda")

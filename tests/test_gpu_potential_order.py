@@ -161,3 +161,21 @@ def test_more_chains_than_subsamples_are_refused(degree):
     with pytest.raises(ValueError, match="subsamples of 4"):
         potential_energy(model, z)
     assert torch.isfinite(potential_energy(model, z[:4])).all()
+
+
+def test_model_data_still_on_its_way_on_another_stream():
+    from numpyro_amd.models import StochasticVolatility, potential_energy
+    r = torch.randn(500, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+    z = 0.1 * torch.ones((3, 502), device="cuda")
+    want = potential_energy(StochasticVolatility(r, noncentred=True), z)
+    data, work = torch.cuda.Stream(), torch.cuda.Stream()
+    late = torch.zeros_like(r)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(data):
+        torch.cuda._sleep(100_000_000)  # some tens of milliseconds
+        late.copy_(r)
+        model = StochasticVolatility(late, noncentred=True)
+    with torch.cuda.stream(work):
+        got = potential_energy(model, z)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
