@@ -185,7 +185,7 @@ diag_lags_kernel(const float* __restrict__ x, int C, int S, int P, int ldx,
       }
     }
     if (t0 < t1) {
-      // w[(u + j) % 8] holds the centred value at t + u + k0 + j
+      // w[(u + j) % 16] holds the centred value at t + u + k0 + j
       auto at = [&](int r) { return r < S ? (double)xs[r * PT + p] - mean : 0.0; };
       double w[kDiagLpt];
 #pragma unroll

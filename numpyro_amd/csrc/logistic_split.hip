@@ -46,13 +46,15 @@
 // The split takes a design whose columns are finite with max |X_d| <= 2^12
 // rms(X_d), so that this is below fp32's own rounding of a typical element, and
 // labels in [0, 1] (|r| <= 1; fp16 ends at |R'| = 2^16).
-// Its number of rows is bounded too: on more than kSplitRows rows per partial
-// sum the fp32 accumulators' own rounding reaches 1e-5 of the gradient
-// (N = 2,000,000, 1024 chains: 9e-6 to 2e-5), and results would differ by it
-// from those of the fp32 MFMA although the split's are no less exact; below
-// kSplitMin rows the rounding of single terms no longer averages out (N = 1000:
-// 2.0e-7 against 1.2e-7) and a launch is mostly latency.  Other designs take
-// the fp32 MFMA in GEMM2 too.
+// Its number of rows is bounded too.  On more than kSplitRows rows per partial
+// sum the fp32 accumulators' own rounding is what a result's error consists of,
+// and the two forms round differently: the split's error is half the fp32 form's
+// (N = 2,000,000, 1024 chains: 4e-6 and 1.4e-5 of the gradient's norm, 12.9 and 16.6
+// ms), but their results differ by the larger, so such designs keep the form that
+// they have had.  Below kSplitMin rows a launch is mostly latency and the split
+// gains little or nothing (256 chains: 16,000 x 55 34.8 against 31.6 us in fp32,
+// 16,000 x 200 62 against 69, 65,536 x 100 80 against 96).  Other designs take the
+// fp32 MFMA in GEMM2 too.
 //
 // Bound: MFMA issue (D = 256: GEMM1 8192 cycles per tile and wave, GEMM2 2560
 // split, 8192 in fp32) plus the epilogue's VALU work, which the fp32 MFMA hardly
