@@ -561,13 +561,14 @@ def model_kernel_name(x_dtype, N, D, C, single=False):
     if x_dtype == "bf16":
         return f"logit_bf16_pipe<{dp}, {'true' if single else 'false'}>"
     if x_dtype == "fp8":
-        if D <= 256 and N >= 65536:
+        few = (C <= 8 and D <= 224) or (C <= 16 and D <= 64)
+        if D <= 256 and N >= 65536 and not few:
             return f"logit_split_kernel<{dp}, fp8>"
         return "logit_partial_f32<XFP8> (VALU tile, e4m3 decoded to fp32)"
     if C <= 16 and D <= 64 and N * D <= (1 << 20):
         return (f"persistent_head_kernel<LogisticChainModel<{32 if D <= 32 else 64}>> "
                 "(a group of wavefronts per chain, autotuned; a launch runs a chunk of iterations)")
-    if D > 256:
+    if D > 256 or (C < 32 and (N < 4000 or (C > 8 and N < 16000) or (C > 16 and D <= 16))):
         return "logit_partial_f32 (VALU tile)"
     if C < 32:
         return f"logit_rows_kernel<{(D + 63) // 64}, {1 if C <= 4 else 2 if C <= 8 else 4}>"

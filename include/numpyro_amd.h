@@ -174,7 +174,8 @@ int nax_model_hier(nax_sampler* h, const float* d_x, const float* d_y, const int
 /* nax_model_logistic with the kernel choice for fp32 storage: 0 = auto
  * (one wavefront per chain in a persistent launch for <= 16 chains on
  * n*d <= 2^20, d <= 64; otherwise, for d <= 256, row tiles on the fp32 matrix
- * cores below 32 chains, the VALU tile kernel or the matrix-core kernel,
+ * cores below 32 chains (the VALU tile kernel on few rows, or few columns and
+ * more than 16 chains), the VALU tile kernel or the matrix-core kernel,
  * whichever the autotuner times faster, up to 128 and the matrix-core kernel
  * above; the VALU tile kernel for 257 <= d <= 320; the matrix-core kernel takes
  * X Z^T in fp32 and X^T R by two fp16 terms of X and three of R where rows, column
@@ -186,8 +187,8 @@ int nax_model_hier(nax_sampler* h, const float* d_x, const float* d_y, const int
  * gradient rounding of 2^-11 instead of 2^-8 per term, and max|X| < 60000).
  * fp8 storage (NAX_X_FP8; the library quantises d_x as nax_fp8_quantize
  * does and keeps the codes): 0 (auto: the matrix cores for d <= 256,
- * n >= 65536 and labels in [0, 1], else the VALU tile kernel with autotuned row
- * splits) or 1 (VALU tile kernel).  Other kernel values with bf16 or fp8
+ * n >= 65536, labels in [0, 1] and more than a few chains, else the VALU tile
+ * kernel) or 1 (VALU tile kernel).  Other kernel values with bf16 or fp8
  * storage, and 4 with fp32 storage, are refused (NAX_EINVAL). */
 int nax_model_logistic_ex(nax_sampler* h, const float* d_x, const float* d_y, int64_t n,
                           int32_t d, double prior_scale, int32_t x_dtype, int32_t kernel);

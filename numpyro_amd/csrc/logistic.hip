@@ -411,7 +411,7 @@ static hipError_t scratch_address(unsigned char** out) {
 // Row splits for `count` chains: the VALU tile kernel's rule (as the
 // handle-based fp32 tile potential uses it), reduced until the partials fit
 // the scratch array; 0 when even one split does not fit.
-static static int noalloc_row_splits(int64_t n, int d, int count) {
+static int noalloc_row_splits(int64_t n, int d, int count) {
   constexpr int BN = 32, BC = 8;
   const int ctiles = (count + BC - 1) / BC;
   const int64_t ntiles = (n + BN - 1) / BN;
@@ -475,6 +475,26 @@ Potential* make_logistic_split(const float* x, const uint8_t* codes, const float
                                int num_chains, bool fp32_products, hipStream_t s,
                                std::string* err);
 
+// The automatic choice for which the VALU tile kernel at its default row splits is
+// the faster one.  Its time goes with the groups of eight chains, the columns and
+// the rows, and its launch is short; the other kernels take more chains at once but
+// have longer tiles.  Device time of a call, tile kernel / the other.
+//
+// fp8 (the other: 128 chains a block on the matrix cores): 8 chains, 200,000 x 20,
+// 60, 160, 200, 250 38 / 71, 54 / 91, 128 / 171, 220 / 219, 256 / 226 us (500,000 x
+// 200 444 / 489, 70,000 x 200 85 / 99); 16 chains x 60 81 / 91, x 100 124 / 119.
+static bool few_chains_fp8(int d, int chains) {
+  return (chains <= 8 && d <= 224) || (chains <= 16 && d <= 64);
+}
+// fp32 (the other: row tiles of 32 on waves of their own, which a short design leaves
+// with a tile or none).  1 chain: 2000 x 65, 256 16 / 17, 24 / 36; 4000 x 65, 256
+// 17 / 15, 25 / 23.  16 chains, x 100: 8000 rows 20 / 25, 16,000 27 / 26.  31 chains of
+// few columns: 150,000 x 2, 16, 32 49 / 51, 58 / 53, 70 / 58 (17 chains 42 / 50, 49 / 52,
+// 60 / 57).
+static bool few_chains_fp32(int64_t n, int d, int chains) {
+  return n < 4000 || (chains > 8 && n < 16000) || (chains > 16 && d <= 16);
+}
+
 // fuse_variant: 0 = auto (fp32: row tiles below 32 chains, else matrix cores), 1 = VALU tile
 // kernel, 2 = matrix cores, 3 = a group of wavefronts per chain.  bf16 always runs on
 // the matrix cores: 0 or 4 keep one X copy (bf16 residuals in X^T R), 2 keeps
@@ -507,12 +527,15 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
   if (!fp8 && (fuse_variant == 3 || (fuse_variant == 0 && num_chains <= 16 && d <= 64 &&
                                      (double)n * d <= (double)(1 << 20))))
     return make_logistic_chain(x, y, n, d, prior_scale, s, err);
-  // fp8: the matrix cores from logistic_split_min_rows() rows on, for any number
-  // of chains (the tile kernel takes 8 chains at a time through a table lookup
-  // per element; a call at 500,000 x 250: 250 chains 15.0 ms against 1.0, 32 chains
-  // 2.24 against 0.68, 1 chain 0.94 against 0.62; 70,000 x 30, 2 chains 0.35 against
-  // 0.22), for labels in [0, 1]
-  bool mfma = fp8 ? fuse_variant == 0 && d <= 256 && n >= logistic_split_min_rows()
+  // fp8: the matrix cores from logistic_split_min_rows() rows on, for labels in
+  // [0, 1], unless few chains are faster on the tile kernel, which takes 8 chains at a
+  // time through a table lookup per element (500,000 x 250, 250 chains 14.9 ms against
+  // 0.95, 32 chains 1.89 against 0.50)
+  const bool tall = d <= 256 && n >= logistic_split_min_rows();
+  const bool few = fuse_variant == 0 && num_chains >= 1 && num_chains < 32 && d <= 256 &&
+                   (fp8 ? tall && few_chains_fp8(d, num_chains)
+                        : few_chains_fp32(n, d, num_chains));
+  bool mfma = fp8 ? fuse_variant == 0 && tall && !few
                   : fuse_variant == 2 || (fuse_variant == 0 && num_chains >= 32 && d <= 256);
   if (fp8 && mfma) {
     const hipError_t e = logistic_split_labels(y, n, s, &mfma);
@@ -532,12 +555,11 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
     *err = "the fp32 logistic tile kernel supports dim <= 320";
     return nullptr;
   }
-  // up to 31 chains: wave-owned row tiles on the fp32 matrix cores (a pass, against
+  // up to 31 chains of a long enough design: wave-owned row tiles on the fp32 matrix cores (a pass, against
   // the tile kernel at its best row split: 581,012 x 55, 1, 8, 16, 31 chains 66, 79,
   // 115, 187 us against 105, 118, 185, 325; 1,000,000 x 256, 1, 16, 31 chains 0.29,
-  // 0.77, 1.49 ms against 1.02, 1.94, 3.83; 2,000 x 100, 4 chains both at the host's
-  // 70).  Its LDS tiles hold 256 columns.
-  if (!fp8 && fuse_variant == 0 && num_chains >= 1 && num_chains < 32 && d <= 256)
+  // 0.77, 1.49 ms against 1.02, 1.94, 3.83).  Its LDS tiles hold 256 columns.
+  if (!fp8 && !few && fuse_variant == 0 && num_chains >= 1 && num_chains < 32 && d <= 256)
     return make_logistic_rows(x, y, n, d, prior_scale);
   auto* p = new LogisticPotential();
   p->x = x;
@@ -560,7 +582,7 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
       return q;
     }
   }
-  if (fuse_variant != 0 || num_chains < 1) return p;
+  if (fuse_variant != 0 || num_chains < 1 || few) return p;
   // Autotuner ("auto" kernel): row splits of the tile kernel (fp8 of few rows, fp32
   // of 257 to 320 columns or 32 to 128 chains), and for 32 <= C <= 128 the tile
   // kernel against the matrix-core kernel, each timed over a

@@ -7,10 +7,14 @@ import bench
 
 @pytest.mark.parametrize("x_dtype, N, D, C, name", [
     ("fp8", 2_000_000, 256, 64, "logit_split_kernel<256, fp8>"),
-    ("fp8", 65_536, 33, 1, "logit_split_kernel<64, fp8>"),
+    ("fp8", 65_536, 33, 17, "logit_split_kernel<64, fp8>"),
+    ("fp8", 65_536, 33, 16, "logit_partial_f32<XFP8>"),
     ("fp8", 65_535, 33, 1024, "logit_partial_f32<XFP8>"),
     ("fp8", 100_000, 257, 1024, "logit_partial_f32<XFP8>"),
     ("fp32", 1000, 26, 4, "persistent_head_kernel<LogisticChainModel<32>>"),
+    ("fp32", 3999, 200, 4, "logit_partial_f32 (VALU tile)"),
+    ("fp32", 15_999, 70, 9, "logit_partial_f32 (VALU tile)"),
+    ("fp32", 1_000_000, 16, 17, "logit_partial_f32 (VALU tile)"),
     ("fp32", 581_012, 55, 1, "logit_rows_kernel<1, 1>"),
     ("fp32", 1_000_000, 256, 31, "logit_rows_kernel<4, 4>"),
     ("fp32", 1_000_000, 130, 8, "logit_rows_kernel<3, 2>"),
