@@ -342,6 +342,7 @@ constexpr int kDiagSlab = 1 << 18;
 // Launch shape and workspace of one call.
 struct DiagPlan {
   int pt, tiles, ng, cap;  // cap: workgroups resident on the chip
+  int first;               // lag passes of the first round
   size_t agg, state, lists, part;  // bytes
   size_t total() const { return agg + state + lists + part; }
 };
@@ -364,8 +365,16 @@ static DiagPlan diag_plan(int C, int S, int P) {
   d.agg = up(sizeof(double) * kAggDoubles * d.ng * cols);
   d.state = up(sizeof(DiagState) * (size_t)P);
   d.lists = up(sizeof(int) * (2 * (size_t)d.tiles + 2));
-  // the first pass, and room for more lags of the tiles that go on
-  d.part = up(std::max(sizeof(double) * kDiagPass * d.ng * cols, (size_t)16 << 20));
+  // One round takes all lags of up to 256 draws where their workgroups fit the chip
+  // at once: they run beside those of the first 32, and another round is three
+  // launches, a copy and a wait (a call on 1 chain x 50, 100 and 200 draws of 60
+  // parameters 47, 48 and 51 us in rounds, 36, 37 and 40 in one; 32, 39 and 53 with
+  // a workgroup per parameter).  More draws leave the finish with more lags in a row
+  // than rounds cost (4 x 1000 x 700 62 us, 102 in one).
+  const int all = std::max(1, (S / 2 * 2 + kDiagPass - 1) / kDiagPass);
+  d.first = all <= 8 && (int64_t)all * d.tiles * d.ng <= d.cap ? all : 1;
+  // the first round, and room for more lags of the tiles that go on
+  d.part = up(std::max(sizeof(double) * kDiagPass * d.first * d.ng * cols, (size_t)16 << 20));
   return d;
 }
 
@@ -382,7 +391,7 @@ static hipError_t diag_launch(const DiagPlan& d, const float* x, int C, int S, i
   hipError_t e = hipFuncSetAttribute((const void*)diag_lags_kernel<PT>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  int nt = d.tiles, base = 0, passes = 1;
+  int nt = d.tiles, base = 0, passes = d.first;
   const int* list = nullptr;
   for (int it = 0;; ++it) {
     const int ng = it == 0 ? d.ng : std::max(1, std::min(C, 2 * d.cap / (nt * passes)));
@@ -394,7 +403,8 @@ static hipError_t diag_launch(const DiagPlan& d, const float* x, int C, int S, i
                             : (int)std::min<size_t>(ng, std::max<size_t>(
                                   1, d.part / (sizeof(double) * kDiagPass * passes * (size_t)nt * PT)));
     int* out = lists + (it & 1) * d.tiles;
-    hipLaunchKernelGGL(diag_zero_kernel, dim3(1), dim3(1), 0, 0, count);
+    const bool last = (base + kDiagPass * passes) / 2 >= S / 2;  // no lags after these
+    if (!last) hipLaunchKernelGGL(diag_zero_kernel, dim3(1), dim3(1), 0, 0, count);
     hipLaunchKernelGGL(diag_lags_kernel<PT>, dim3((nt * fit + 7) / 8 * 8, passes),
                        dim3(kDiagThreads), lds, 0, x, C, S, P, ldx, list, nt, fit, base, part,
                        it == 0 ? agg : nullptr);
@@ -404,7 +414,7 @@ static hipError_t diag_launch(const DiagPlan& d, const float* x, int C, int S, i
     if (e != hipSuccess) return e;
     base += kDiagPass * passes;
     int n = 0;
-    if (base / 2 < S / 2) {
+    if (!last) {
       e = hipMemcpyAsync(&n, count, sizeof(int), hipMemcpyDeviceToHost, 0);
       if (e != hipSuccess) return e;
     }
