@@ -475,8 +475,8 @@ Potential* make_logistic_split(const float* x, const uint8_t* codes, const float
                                int num_chains, bool fp32_products, hipStream_t s,
                                std::string* err);
 
-// The automatic choice for which the VALU tile kernel at its default row splits is
-// the faster one.  Its time goes with the groups of eight chains, the columns and
+// The automatic choice for which the VALU tile kernel, without its autotuner, is the
+// faster one.  Its time goes with the groups of eight chains, the columns and
 // the rows, and its launch is short; the other kernels take more chains at once but
 // have longer tiles.  Device time of a call, tile kernel / the other.
 //
@@ -582,6 +582,12 @@ Potential* make_logistic(const float* x, const float* y, int64_t n, int d, doubl
       return q;
     }
   }
+  // 1024 blocks instead of 2048 on the shorter of these designs: a block of one or two
+  // tiles costs its start (fp32, 17 chains, 32,000 x 4 24 -> 21 us, 31 chains, 15,000 x
+  // 100 37 -> 31, but x 256, 17 chains 63 -> 73; fp8, 1 chain, 70,000 x 160 71 -> 55,
+  // 200,000 x 160 136 -> 117, but x 200 210 -> 234; 500,000 x 60 91 -> 111).
+  if (few && (fp8 ? n < 300000 && d <= 160 : n < 100000 && d <= 128))
+    p->rb_pick = 1024 / ((num_chains + 7) / 8);
   if (fuse_variant != 0 || num_chains < 1 || few) return p;
   // Autotuner ("auto" kernel): row splits of the tile kernel (fp8 of few rows, fp32
   // of 257 to 320 columns or 32 to 128 chains), and for 32 <= C <= 128 the tile

@@ -13,11 +13,17 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("x_dtype, N, D, C", [
     ("fp32", 1000, 256, 16), ("fp32", 3999, 65, 1), ("fp32", 500, 3, 31), ("fp32", 15999, 70, 9),
-    ("fp32", 15999, 256, 31), ("fp32", 70000, 16, 17), ("fp8", 65536, 20, 1),
-    ("fp8", 70001, 224, 8), ("fp8", 70001, 64, 16)])
+    ("fp32", 15999, 256, 31), ("fp32", 100001, 16, 17), ("fp8", 300001, 20, 1),
+    ("fp8", 65536, 224, 8), ("fp8", 300001, 64, 16)])
 def test_tile_kernel_where_it_is_faster(x_dtype, N, D, C):
     X, y, z = _data(N, D, C, N + D)
     assert torch.equal(_grad(X, y, z, x_dtype, "auto"), _grad(X, y, z, x_dtype, "tile"))
+
+
+@pytest.mark.parametrize("x_dtype, N, D, C", [("fp32", 32001, 4, 17), ("fp32", 99999, 16, 31),
+                                              ("fp8", 65536, 20, 1), ("fp8", 70001, 64, 16)])
+def test_tile_kernel_at_half_the_row_splits(x_dtype, N, D, C):
+    _check(*_data(N, D, C, N + D), x_dtype=x_dtype, kernel="auto")
 
 
 @pytest.mark.parametrize("n, d, C", [(4000, 65, 1), (4033, 129, 8), (4127, 256, 5), (16000, 192, 9),
