@@ -184,7 +184,8 @@ __global__ void ecs_reduce_kernel(const double* part, int nsplit, int64_t len, d
 // L2) serves all of them; a workgroup per chain read it once per chain, inside
 // the evaluation and after all of its gathers.  Threads: 256 columns of H
 // (symmetric, so column reads are coalesced) times 4 quarters of its rows, 16
-// loads in flight each.  1024 chains, d = 256: 7 us.
+// loads in flight each.  1024 chains, d = 256: 13 us
+// behind evaluations whose rows have taken L2.
 constexpr int kProxyChains = 4, kProxyParts = 4;
 __global__ __launch_bounds__(kEcsThreads * kProxyParts) void ecs_proxy_kernel(
     EcsArgs a, const float* __restrict__ z, int ldz, int C, const int* act, const int* nact,

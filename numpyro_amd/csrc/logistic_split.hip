@@ -63,7 +63,7 @@
 // runs beside the other's epilogue.  Main kernel, both products in fp32 and
 // split: 581,012 x 55, 256 chains 412 and 319 us (281 with one term below R's grid);
 // 500,000 x 250, 256 chains 1.06 and 0.85 ms (0.76); fp8 500,000 x 250, 250 chains
-// 13.6 ms on the VALU tile kernel and 0.90 (0.81).  2,000,000 x 256, 1024 chains
+// 13.3 ms on the VALU tile kernel and 0.94 (0.81).  2,000,000 x 256, 1024 chains
 // (fp32 form) 17.0 ms with the epilogue between the products, 16.5 as here.
 #include <hip/hip_runtime.h>
 
