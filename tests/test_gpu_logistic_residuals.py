@@ -71,6 +71,28 @@ def test_rare_events_keep_their_bits(D, rate, x_dtype, C):
     assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
 
 
+@pytest.mark.parametrize("x_dtype, C", [("fp32", 130), ("fp8", 33)])
+@pytest.mark.parametrize("intercept", [-4.0, -7.0, -9.0])
+def test_intercept_and_binary_columns(intercept, x_dtype, C):
+    """Eight patterns of three binary columns beside an intercept; K = 4 terms of a
+    logit are not zero."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    X = (torch.rand((N, 4), generator=g, device="cuda") < 0.3).float()
+    X[:, 0] = 1.0
+    beta = torch.tensor([intercept, 0.5, -0.7, 1.1], device="cuda")
+    y = (torch.rand(N, generator=g, device="cuda") < torch.sigmoid(X @ beta)).float()
+    z = beta + 0.1 * torch.randn((C, 4), generator=g, device="cuda")
+    got = _grad(X, y, z, x_dtype, "auto")
+    x, z64 = X.double(), z.double()
+    l = x @ z64.T
+    r = torch.sigmoid(l) - y.double()[:, None]
+    want = r.T.contiguous() @ x + z64
+    M = float((x @ z64.abs().T).max())
+    eps = (5 * M + 1.5 * math.log(2) * 1.4427 * M + 6 + 5 * 512 / 32) * 2.0 ** -24
+    bound = eps * (r.abs().T.contiguous() @ x) + 2.0 ** -23 * z64.abs() + 1e-9
+    assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
+
+
 def _single_entries(C):
     """64 columns of one number each, 24 bits long, in rows of their own."""
     g = torch.Generator(device="cuda").manual_seed(5)
